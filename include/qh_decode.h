@@ -277,7 +277,9 @@ int qh_decode_token(qh_engine* e, int tok, float* logits, int* argmax_out);
  * greedily generate up to n_new ids, stopping before emitting `eos` (eos < 0:
  * never).  out_ids receives the generated ids, *n_out their count.  The token
  * feedback stays on the device: one persistent launch (or one graph replay per
- * token) and no host round trip between tokens. */
+ * token) and no host round trip between tokens.  A prompt's tokens but the last
+ * run in groups (one read of the weights per group of up to 512 tokens) where
+ * that is faster; the state they leave is the token-by-token state bit for bit. */
 int qh_generate(qh_engine* e, const int* prompt, int n_prompt, int n_new, int eos, int* out_ids,
                 int* n_out);
 /* Tokens processed so far (DecodeState::pos). */

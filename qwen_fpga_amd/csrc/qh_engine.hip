@@ -19,6 +19,7 @@
 #include "qh_common.hpp"
 #include "qh_kernels.hpp"
 #include "qh_layout.hpp"
+#include "qh_prefill.hpp"
 
 using namespace qh;
 
@@ -81,6 +82,9 @@ struct qh_engine {
   unsigned poll_limit = 1u << 20;  // failed polls before a hand-over wait gives up (QH_POLL_LIMIT)
   bool broken = false;             // a launch returned QH_EDEVICE: decode refused until reset
   int fallbacks = 0;               // cooperative launches refused (each switched the engine to the graph path)
+  // Grouped prompt path (qh_prefill.hip): one allocation, made by the first prompt that takes it.
+  char* pf = nullptr;
+  bool pf_off = false;             // its allocation failed: prompts are fed token by token
   bool dn_lds = false;             // the persistent kernel keeps the DeltaNet state in LDS (enough workgroups)
 };
 
@@ -501,11 +505,12 @@ constexpr int kUseGraph = 1000;
 
 // One persistent launch: the prompt (already in prompt_dev) through the
 // run_hls loop, n_new greedy tokens at most, token feedback on the device.
-int run_persist(qh_engine* e, int tok0, int n_prompt, int n_new, int eos, bool with_logits, StepCtl* out) {
+// step0: prompt tokens already processed; tok0 is the next one.
+int run_persist(qh_engine* e, int tok0, int step0, int n_prompt, int n_new, int eos, bool with_logits, StepCtl* out) {
   QH_TRY(ensure_prog(e));
   hipStream_t s = e->stream;
-  // tags of this launch: tag_base + k * kTagsPerToken + stage, k < n_prompt + n_new
-  const uint64_t need = ((uint64_t)n_prompt + (uint64_t)n_new + 1) * kTagsPerToken;
+  // tags of this launch: tag_base + k * kTagsPerToken + stage, k < n_prompt - step0 + n_new
+  const uint64_t need = ((uint64_t)(n_prompt - step0) + (uint64_t)n_new + 1) * kTagsPerToken;
   if ((uint64_t)e->tag_next + need > 0xFFFFFFFFull) {   // tags would wrap: clear the arena
     QH_HIP(hipMemsetAsync(e->arena, 0, sizeof(uint64_t) * e->arena_pairs, s));
     e->tag_next = 1;
@@ -515,6 +520,7 @@ int run_persist(qh_engine* e, int tok0, int n_prompt, int n_new, int eos, bool w
   c.tok = tok0;
   c.pos = e->host_pos;
   c.argmax = e->last_argmax;
+  c.step = step0;
   c.n_prompt = n_prompt;
   c.n_new = n_new;
   c.eos = eos;
@@ -631,6 +637,206 @@ int get_graph(qh_engine* e, bool with_logits, bool advance, hipGraphExec_t* out)
   return QH_OK;
 }
 
+// ---- prompts in groups (qh_prefill.hip) ----
+// Device buffers of a group of kPfGroup tokens, carved from one allocation.
+struct PfBufs {
+  float *h, *y, *o, *qk, *v, *gates, *qf, *kf, *xs;
+  char *x, *x2;
+  size_t bytes;
+  explicit PfBufs(char* base) {
+    size_t used = 0;
+    auto take = [&](size_t n) {
+      char* p = base + used;
+      used += (n + 255) & ~(size_t)255;
+      return p;
+    };
+    auto f = [&](size_t n) { return reinterpret_cast<float*>(take(4 * n)); };
+    constexpr size_t G = kPfGroup;
+    h = f(G * kHidden);                    // residual stream
+    y = f(G * (kConvDim + kZDim));         // qkv | silu(z); q || gate, k, v; W8A8: act
+    o = f(G * kLH * kLV);                  // delta-rule output; W8A8: attention context
+    qk = f(G * 2 * kLH * kLK);             // the scan's q, k; v; exp(g), beta
+    v = f(G * kLH * kLV);
+    gates = f(G * 2 * kLH);
+    qf = f((G + kPfTile) * kNH * kHD);     // query fragments (the group may start inside a tile)
+    kf = f((size_t)kPfMaxPos * kKVProj);   // key fragments of every position
+    xs = f(G);
+    x = take(G * 4 * 4096);                // activation fragments (the widest: fp32, 4 chunks of 16 per lane)
+    x2 = take(G * 4 * 4096);               // W8A16: the MLP activation's
+    bytes = used;
+  }
+};
+
+// The shortest run of prompt tokens that goes as a group.  A group of 4 tokens takes 2.1 ms in W8A8 and
+// 5.2 ms in W8A16 (every weight byte read once, 240 launches), hardly more up to 64; a token by itself
+// takes 0.43 ms on the persistent executor and 0.75 ms on the graph executor.
+int prefill_min(const qh_engine* e) {
+  if (e->exec == QH_EXEC_PERSISTENT) return e->mode == M_W8A8 ? 6 : 13;
+  return e->mode == M_W8A8 ? 4 : 8;
+}
+
+// How many of a prompt's first tokens run in groups: all but the last (the executor runs it, with the
+// LM head), up to the positions the grouped attention covers.
+int prefill_tokens(const qh_engine* e, int n_prompt) {
+  int n = n_prompt - 1;
+  if (n > kPfMaxPos - e->host_pos) n = kPfMaxPos - e->host_pos;
+  return n < prefill_min(e) || e->pf_off ? 0 : n;
+}
+
+// One group: M tokens of prompt_dev from `first`, at positions host_pos ..; all layers in order.
+int prefill_group(qh_engine* e, const PfBufs& b, int first, int M) {
+  hipStream_t s = e->stream;
+  const int mode = e->mode, pos0 = e->host_pos;
+  int li = 0, fi = 0;
+  for (int l = 0; l < kLayers; ++l) {
+    const bool lin = is_linear(l);
+    PfNorm nm;
+    nm.h = b.h;
+    if (l == 0) {
+      nm.h_out = b.h;
+      nm.emb = i8p(e, kLayers, R_EMBED);
+      nm.emb_s = scp(e, kLayers, R_EMBED);
+      nm.ids = e->prompt_dev + first;
+    }
+    nm.nw = lanep(e, l, R_IN_LN);
+    nm.eps = kEps;
+    nm.x = b.x;
+    nm.xs = b.xs;
+    nm.M = M;
+    if (lin) {
+      nm.gw = lanep(e, l, R_B);   // wb rows, then the wa rows (consecutive in lanes)
+      nm.A_log = f32p(e, l, R_ALOG);
+      nm.dt_bias = f32p(e, l, R_DTB);
+      nm.gates = b.gates;
+    }
+    QH_HIP(pf_norm(nm, mode, s));
+    PfGemm g;
+    g.x = b.x;
+    g.xs = b.xs;
+    g.out = b.y;
+    g.M = M;
+    PfGemm r;   // the projection back to the residual stream
+    r.x = b.x;
+    r.xs = b.xs;
+    r.out = b.h;
+    r.ld = kHidden;
+    r.rows = kHidden;
+    r.M = M;
+    if (lin) {
+      g.nseg = 2;
+      g.w[0] = i8p(e, l, R_QKV), g.sw[0] = scp(e, l, R_QKV);
+      g.w[1] = i8p(e, l, R_Z), g.sw[1] = scp(e, l, R_Z), g.row0[1] = kConvDim;
+      g.rows = g.ld = kConvDim + kZDim;
+      QH_HIP(pf_gemm(g, kHidden, PF_INPROJ, mode, s));
+      PfConv c;
+      c.y = b.y;
+      c.taps = f32p(e, l, R_CONV);
+      c.state = e->conv + (size_t)li * kConvDim * kConvK;
+      c.qk = b.qk;
+      c.v = b.v;
+      c.M = M;
+      QH_HIP(pf_conv(c, s));
+      PfScan d;
+      d.qk = b.qk;
+      d.v = b.v;
+      d.gates = b.gates;
+      d.S = e->rec + (size_t)li * kLH * kLK * kLV;
+      d.o = b.o;
+      d.M = M;
+      QH_HIP(pf_scan(d, s));
+      PfGated gt;
+      gt.o = b.o;
+      gt.y = b.y;
+      gt.nw = f32p(e, l, R_LNORM);
+      gt.eps = kEps;
+      gt.x = b.x;
+      gt.xs = b.xs;
+      gt.conv_state = e->conv + (size_t)li * kConvDim * kConvK;
+      gt.M = M;
+      QH_HIP(pf_gated(gt, mode, s));
+      r.w[0] = i8p(e, l, R_OUTP), r.sw[0] = scp(e, l, R_OUTP);
+      QH_HIP(pf_gemm(r, kLH * kLV, PF_RESID, mode, s));
+      ++li;
+    } else {
+      g.nseg = 3;
+      g.w[0] = i8p(e, l, R_QP), g.sw[0] = scp(e, l, R_QP);
+      g.w[1] = i8p(e, l, R_KP), g.sw[1] = scp(e, l, R_KP), g.row0[1] = kQProj;
+      g.w[2] = i8p(e, l, R_VP), g.sw[2] = scp(e, l, R_VP), g.row0[2] = kQProj + kKVProj;
+      g.rows = g.ld = kQProj + 2 * kKVProj;
+      QH_HIP(pf_gemm(g, kHidden, PF_STORE, mode, s));
+      PfAttn a;
+      a.qkv = b.y;
+      a.qn = f32p(e, l, R_QN);
+      a.kn = f32p(e, l, R_KN);
+      a.rope = e->rope;
+      a.kc = e->kc + (size_t)fi * e->max_ctx * kKVProj;
+      a.vc = e->vc + (size_t)fi * e->max_ctx * kKVProj;
+      a.qf = b.qf;
+      a.kf = b.kf;
+      a.og = mode == M_W8A8 ? b.o : reinterpret_cast<float*>(b.x);
+      a.eps = kEps;
+      a.pos0 = pos0;
+      a.M = M;
+      QH_HIP(pf_qk(a, s));
+      QH_HIP(pf_attn(a, mode, s));
+      if (mode == M_W8A8) QH_HIP(pf_quant(b.x, b.xs, b.o, kNH * kHD, M, s));
+      r.w[0] = i8p(e, l, R_OP), r.sw[0] = scp(e, l, R_OP);
+      QH_HIP(pf_gemm(r, kNH * kHD, PF_RESID, mode, s));
+      ++fi;
+    }
+    PfNorm pn;
+    pn.h = b.h;
+    pn.nw = lanep(e, l, R_POST_LN);
+    pn.eps = kEps;
+    pn.x = b.x;
+    pn.xs = b.xs;
+    pn.M = M;
+    QH_HIP(pf_norm(pn, mode, s));
+    PfGemm m;
+    m.nseg = 2;
+    m.w[0] = i8p(e, l, R_GATE), m.sw[0] = scp(e, l, R_GATE);
+    m.w[1] = i8p(e, l, R_UP), m.sw[1] = scp(e, l, R_UP);
+    m.rows = 2 * kInter;
+    m.x = b.x;
+    m.xs = b.xs;
+    m.out = mode == M_W8A8 ? b.y : reinterpret_cast<float*>(b.x2);
+    m.ld = kInter;
+    m.M = M;
+    QH_HIP(pf_gemm(m, kHidden, PF_SWIGLU, mode, s));
+    if (mode == M_W8A8) QH_HIP(pf_quant(b.x2, b.xs, b.y, kInter, M, s));
+    r.x = b.x2;
+    r.w[0] = i8p(e, l, R_DOWN), r.sw[0] = scp(e, l, R_DOWN);
+    QH_HIP(pf_gemm(r, kInter, PF_RESID, mode, s));
+  }
+  return QH_OK;
+}
+
+// The first n tokens of prompt_dev in groups; *done receives how many ran (0: fed one by one).  A
+// failed launch leaves the state between two tokens' states: decoding is refused until a reset.
+int run_prefill(qh_engine* e, int n, int* done) {
+  *done = 0;
+  if (n <= 0) return QH_OK;
+  if (e->pf == nullptr) {
+    if (hipMalloc(reinterpret_cast<void**>(&e->pf), PfBufs(nullptr).bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      e->pf = nullptr;
+      e->pf_off = true;
+      return QH_OK;
+    }
+  }
+  const PfBufs b(e->pf);
+  for (int i = 0; i < n; i += kPfGroup) {
+    const int M = n - i < kPfGroup ? n - i : kPfGroup;
+    if (const int st = prefill_group(e, b, i, M); st != QH_OK) {
+      e->broken = true;
+      return st;
+    }
+    e->host_pos += M;
+  }
+  *done = n;
+  return QH_OK;
+}
+
 void release(qh_engine* e) {
   if (!e) return;
   if (e->stream) (void)hipStreamSynchronize(e->stream);
@@ -641,7 +847,7 @@ void release(qh_engine* e) {
   void* bufs[] = {e->blob, e->rec, e->conv, e->kc, e->vc, e->h, e->convd, e->zb, e->gb, e->o, e->act,
                   e->og, e->qkv, e->pm, e->pl, e->pacc, e->rope, e->logits, e->part_val,
                   e->part_idx, e->ctl, e->prompt_dev, e->out_dev, e->prog[0], e->prog[1], e->arena,
-                  e->abort_dev, e->lanes};
+                  e->abort_dev, e->lanes, e->pf};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (hipEvent_t ev : e->launch_ev)
@@ -868,7 +1074,7 @@ int qh_decode_token(qh_engine* e, int tok, float* logits, int* argmax_out) {
   if (e->exec == QH_EXEC_PERSISTENT) {   // one token = a prompt of one, no new tokens
     QH_HIP(hipMemcpyAsync(e->prompt_dev, &tok, sizeof(int), hipMemcpyHostToDevice, e->stream));
     StepCtl c;
-    const int st = run_persist(e, tok, 1, 0, -1, logits != nullptr, &c);
+    const int st = run_persist(e, tok, 0, 1, 0, -1, logits != nullptr, &c);
     if (st != kUseGraph) {
       QH_TRY(st);
       if (logits) QH_HIP(hipMemcpy(logits, e->logits, sizeof(float) * kVocab, hipMemcpyDeviceToHost));
@@ -902,9 +1108,11 @@ int qh_generate(qh_engine* e, const int* prompt, int n_prompt, int n_new, int eo
   hipStream_t s = e->stream;
   QH_HIP(hipMemcpyAsync(e->prompt_dev, prompt, sizeof(int) * (size_t)n_prompt, hipMemcpyHostToDevice, s));
   QH_HIP(hipStreamSynchronize(s));
+  int step0 = 0;   // prompt tokens run as groups; the rest, the last one at least, one by one
+  QH_TRY(run_prefill(e, prefill_tokens(e, n_prompt), &step0));
   if (e->exec == QH_EXEC_PERSISTENT) {
     StepCtl c;
-    const int st = run_persist(e, prompt[0], n_prompt, n_new, eos, false, &c);
+    const int st = run_persist(e, prompt[step0], step0, n_prompt, n_new, eos, false, &c);
     if (st != kUseGraph) {
       QH_TRY(st);
       if (c.n_out > 0)
@@ -915,8 +1123,9 @@ int qh_generate(qh_engine* e, const int* prompt, int n_prompt, int n_new, int eo
   }
   hipGraphExec_t g;
   QH_TRY(get_graph(e, false, true, &g));
-  QH_HIP(launch_init_gen(e->ctl, prompt[0], n_prompt, n_new, eos, s));
-  for (int i = 0; i < n_prompt + n_new; ++i) QH_HIP(hipGraphLaunch(g, s));
+  if (step0 > 0) QH_HIP(launch_set_int(&e->ctl->pos, e->host_pos, s));
+  QH_HIP(launch_init_gen(e->ctl, prompt[step0], step0, n_prompt, n_new, eos, s));
+  for (int i = step0; i < n_prompt + n_new; ++i) QH_HIP(hipGraphLaunch(g, s));
   StepCtl c;
   QH_HIP(hipMemcpyAsync(&c, e->ctl, sizeof c, hipMemcpyDeviceToHost, s));
   QH_HIP(hipStreamSynchronize(s));

@@ -447,9 +447,9 @@ hipError_t launch_bump_pos(StepCtl* ctl, hipStream_t s) {
   return hipGetLastError();
 }
 
-__global__ void init_gen_kernel(StepCtl* c, int tok0, int n_prompt, int n_new, int eos) {
+__global__ void init_gen_kernel(StepCtl* c, int tok0, int step0, int n_prompt, int n_new, int eos) {
   c->tok = tok0;
-  c->step = 0;
+  c->step = step0;
   c->n_prompt = n_prompt;
   c->n_new = n_new;
   c->n_out = 0;
@@ -457,8 +457,8 @@ __global__ void init_gen_kernel(StepCtl* c, int tok0, int n_prompt, int n_new, i
   c->done = 0;
   c->err = 0;
 }
-hipError_t launch_init_gen(StepCtl* ctl, int tok0, int n_prompt, int n_new, int eos, hipStream_t s) {
-  init_gen_kernel<<<1, 1, 0, s>>>(ctl, tok0, n_prompt, n_new, eos);
+hipError_t launch_init_gen(StepCtl* ctl, int tok0, int step0, int n_prompt, int n_new, int eos, hipStream_t s) {
+  init_gen_kernel<<<1, 1, 0, s>>>(ctl, tok0, step0, n_prompt, n_new, eos);
   return hipGetLastError();
 }
 

@@ -304,6 +304,6 @@ hipError_t launch_dn_gather(float* convd, float* gb, const float* q, const float
                             const float* beta, float gs, float bs, int nq, int nv, int nh, hipStream_t s);
 hipError_t launch_set_floats(float* dst, const Floats64& v, int n, hipStream_t s);
 hipError_t launch_bump_pos(StepCtl* ctl, hipStream_t s);
-hipError_t launch_init_gen(StepCtl* ctl, int tok0, int n_prompt, int n_new, int eos, hipStream_t s);
+hipError_t launch_init_gen(StepCtl* ctl, int tok0, int step0, int n_prompt, int n_new, int eos, hipStream_t s);
 
 }  // namespace qh

@@ -1,0 +1,90 @@
+"""Prompts run in groups (qh_prefill.hip) leave what feeding them token by token leaves, bit for
+bit: the recurrent, conv and KV state, the next token and its logits.  Lengths at the edges of the
+MFMA tile (16 tokens), of the group (512), of the positions the grouped attention covers (2048),
+and prompts that start inside a tile.  The prompt's last token always runs on the executor, so n
+tokens take the grouped path for n - 1 of them."""
+import numpy as np
+import pytest
+
+from conftest import assert_bitwise, rng
+from test_gpu_engine import d2h
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(e, n, ctx):
+    return [d2h(e.device_ptr(1), (18, 16, 128, 128)), d2h(e.device_ptr(2), (18, 6144, 4)),
+            d2h(e.device_ptr(3), (6, ctx, 512))[:, :n], d2h(e.device_ptr(4), (6, ctx, 512))[:, :n]]
+
+
+def _check(q, e, parts, ctx):
+    """The prompts `parts` one after another, fed whole and token by token."""
+    n = sum(len(p) for p in parts)
+    e.reset()
+    for p in parts:
+        for t in p:
+            am, _ = e.decode_token(t)
+    want, lw = _state(e, n, ctx), e.decode_token(7, want_logits=True)[1]
+    e.reset()
+    for p in parts:
+        assert e.generate(p, 0) == []
+    assert e.pos == n and e.last_argmax == am
+    got, lg = _state(e, n, ctx), e.decode_token(7, want_logits=True)[1]
+    for a, b, what in zip(got, want, ("recurrent state", "conv state", "k cache", "v cache")):
+        assert_bitwise(a, b, f"{what}, prompts {[len(p) for p in parts]}")
+    assert_bitwise(lg, lw, "next logits")
+
+
+@pytest.mark.parametrize("mode", [0, 1], ids=["w8a16", "w8a8"])
+@pytest.mark.parametrize("exec_kind", ["graph", "persistent"])
+def test_prompt_in_groups_equals_token_by_token(q, blob, torch_cuda, mode, exec_kind):
+    ctx = 600
+    e = q.Engine(blob, max_ctx=ctx, mode=mode)
+    try:
+        e.set_exec(q.EXEC_GRAPH if exec_kind == "graph" else q.EXEC_PERSISTENT)
+        r = rng(77 + mode)
+        ids = lambda n: r.integers(0, q.VOCAB, size=n).astype(np.int32).tolist()
+        lens = [[14], [16], [17], [18], [66], [3, 20], [21, 40, 2, 15]]
+        if exec_kind == "persistent":
+            lens += [[129], [513], [514], [30, 530]]
+        for ls in lens:
+            _check(q, e, [ids(n) for n in ls], ctx)
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("mode", [0, 1], ids=["w8a16", "w8a8"])
+def test_prompt_past_the_short_contexts(q, blob, torch_cuda, mode):
+    """A prompt that ends past 2048 positions: the groups stop there."""
+    ctx = 2080
+    e = q.Engine(blob, max_ctx=ctx, mode=mode)
+    try:
+        e.set_exec(q.EXEC_PERSISTENT)
+        ids = rng(9).integers(0, q.VOCAB, size=2061).astype(np.int32).tolist()
+        _check(q, e, [ids], ctx)
+    finally:
+        e.close()
+
+
+def test_generation_after_a_grouped_prompt(q, blob, torch_cuda):
+    """Greedy ids, eos and the position after a grouped prompt equal those of a host loop."""
+    ctx = 128
+    e = q.Engine(blob, max_ctx=ctx, mode=q.MODE_W8A8)
+    try:
+        ids = rng(3).integers(0, q.VOCAB, size=70).astype(np.int32).tolist()
+        cur = None
+        for t in ids:
+            cur, _ = e.decode_token(t)
+        want = []
+        for _ in range(12):
+            want.append(cur)
+            cur, _ = e.decode_token(cur)
+        for ex in (q.EXEC_GRAPH, q.EXEC_PERSISTENT):
+            e.set_exec(ex)
+            e.reset()
+            assert e.generate(ids, 12) == want and e.pos == 82
+            e.reset()
+            first = want.index(want[5])
+            assert e.generate(ids, 12, eos=want[5]) == want[:first] and e.pos == 70 + first
+    finally:
+        e.close()
