@@ -82,8 +82,13 @@ struct qh_engine {
   unsigned poll_limit = 1u << 20;  // failed polls before a hand-over wait gives up (QH_POLL_LIMIT)
   bool broken = false;             // a launch returned QH_EDEVICE: decode refused until reset
   int fallbacks = 0;               // cooperative launches refused (each switched the engine to the graph path)
-  // Grouped prompt path (qh_prefill.hip): one allocation, made by the first prompt that takes it.
-  char* pf = nullptr;
+  // Grouped prompt path (qh_prefill.hip), made by the first prompt that takes it: the buffers of
+  // up to kPfSlots groups, a stream for each slot after the first (which runs on `stream`), and
+  // per slot and layer the event that its group's state of that layer is complete.
+  char* pf[kPfSlots] = {};
+  int pf_cap[kPfSlots] = {};       // tokens the slot's buffers hold
+  hipStream_t pf_stream[kPfSlots] = {};
+  hipEvent_t pf_ev[kPfSlots][kLayers + 1] = {};   // (the last: the group is complete)
   bool pf_off = false;             // its allocation failed: prompts are fed token by token
   bool dn_lds = false;             // the persistent kernel keeps the DeltaNet state in LDS (enough workgroups)
 };
@@ -638,12 +643,12 @@ int get_graph(qh_engine* e, bool with_logits, bool advance, hipGraphExec_t* out)
 }
 
 // ---- prompts in groups (qh_prefill.hip) ----
-// Device buffers of a group of kPfGroup tokens, carved from one allocation.
+// Device buffers of a group of up to G tokens (a multiple of 32), carved from one allocation.
 struct PfBufs {
   float *h, *y, *o, *qk, *v, *gates, *qf, *kf, *xs;
   char *x, *x2;
   size_t bytes;
-  explicit PfBufs(char* base) {
+  PfBufs(char* base, size_t G) {
     size_t used = 0;
     auto take = [&](size_t n) {
       char* p = base + used;
@@ -651,7 +656,6 @@ struct PfBufs {
       return p;
     };
     auto f = [&](size_t n) { return reinterpret_cast<float*>(take(4 * n)); };
-    constexpr size_t G = kPfGroup;
     h = f(G * kHidden);                    // residual stream
     y = f(G * (kConvDim + kZDim));         // qkv | silu(z); q || gate, k, v; W8A8: act
     o = f(G * kLH * kLV);                  // delta-rule output; W8A8: attention context
@@ -667,12 +671,12 @@ struct PfBufs {
   }
 };
 
-// The shortest run of prompt tokens that goes as a group.  A group of 4 tokens takes 2.1 ms in W8A8 and
-// 5.2 ms in W8A16 (every weight byte read once, 240 launches), hardly more up to 64; a token by itself
-// takes 0.43 ms on the persistent executor and 0.75 ms on the graph executor.
+// The shortest run of prompt tokens that goes as a group.  A group takes 1.6 ms in W8A8 and 2.6 ms in
+// W8A16 at 4 to 32 tokens (240 launches, every weight byte read once); a token by itself takes 0.42 ms
+// on the persistent executor and 0.75 ms on the graph executor.
 int prefill_min(const qh_engine* e) {
-  if (e->exec == QH_EXEC_PERSISTENT) return e->mode == M_W8A8 ? 6 : 13;
-  return e->mode == M_W8A8 ? 4 : 8;
+  if (e->exec == QH_EXEC_PERSISTENT) return e->mode == M_W8A8 ? 5 : 7;
+  return e->mode == M_W8A8 ? 3 : 4;
 }
 
 // How many of a prompt's first tokens run in groups: all but the last (the executor runs it, with the
@@ -683,9 +687,23 @@ int prefill_tokens(const qh_engine* e, int n_prompt) {
   return n < prefill_min(e) || e->pf_off ? 0 : n;
 }
 
-// One group: M tokens of prompt_dev from `first`, at positions host_pos ..; all layers in order.
-int prefill_group(qh_engine* e, const PfBufs& b, int first, int M) {
-  hipStream_t s = e->stream;
+// Tokens per group of a prompt of n (at most kPfMaxPos): one group up to 512 tokens, above that two
+// halves, the second one layer behind the first on a stream of its own.  The two overlap (1024
+// tokens: 6.0 ms in W8A8 where one group after the other takes 8.4), but each is a chain of 240
+// launches: two of 256 took as long as one of 512 (4.1 ms).  A third stream made each wait between
+// groups slower by hundreds of microseconds, so there are never more than two.
+int prefill_group_size(int n) {
+  static_assert(2 * kPfGroup >= kPfMaxPos, "two groups hold every prompt");
+  return n <= 512 ? n : ((n + 1) / 2 + 31) & ~31;
+}
+
+// One group: M tokens of prompt_dev from `first`, at positions host_pos ..; all layers in order, on
+// slot `slot`'s stream.  Where a layer reads what the group before (slot `prev`, -1: none in flight)
+// leaves -- conv history and recurrent state, cache rows -- it waits for that group's event of the
+// layer; everything else of the two groups overlaps.  `events`: a group follows.
+int prefill_group(qh_engine* e, int slot, int prev, bool events, int first, int M) {
+  const PfBufs b(e->pf[slot], (size_t)e->pf_cap[slot]);
+  hipStream_t s = e->pf_stream[slot];
   const int mode = e->mode, pos0 = e->host_pos;
   int li = 0, fi = 0;
   for (int l = 0; l < kLayers; ++l) {
@@ -728,6 +746,7 @@ int prefill_group(qh_engine* e, const PfBufs& b, int first, int M) {
       g.w[1] = i8p(e, l, R_Z), g.sw[1] = scp(e, l, R_Z), g.row0[1] = kConvDim;
       g.rows = g.ld = kConvDim + kZDim;
       QH_HIP(pf_gemm(g, kHidden, PF_INPROJ, mode, s));
+      if (prev >= 0) QH_HIP(hipStreamWaitEvent(s, e->pf_ev[prev][l], 0));
       PfConv c;
       c.y = b.y;
       c.taps = f32p(e, l, R_CONV);
@@ -754,6 +773,7 @@ int prefill_group(qh_engine* e, const PfBufs& b, int first, int M) {
       gt.conv_state = e->conv + (size_t)li * kConvDim * kConvK;
       gt.M = M;
       QH_HIP(pf_gated(gt, mode, s));
+      if (events) QH_HIP(hipEventRecord(e->pf_ev[slot][l], s));
       r.w[0] = i8p(e, l, R_OUTP), r.sw[0] = scp(e, l, R_OUTP);
       QH_HIP(pf_gemm(r, kLH * kLV, PF_RESID, mode, s));
       ++li;
@@ -777,7 +797,9 @@ int prefill_group(qh_engine* e, const PfBufs& b, int first, int M) {
       a.eps = kEps;
       a.pos0 = pos0;
       a.M = M;
+      if (prev >= 0) QH_HIP(hipStreamWaitEvent(s, e->pf_ev[prev][l], 0));
       QH_HIP(pf_qk(a, s));
+      if (events) QH_HIP(hipEventRecord(e->pf_ev[slot][l], s));
       QH_HIP(pf_attn(a, mode, s));
       if (mode == M_W8A8) QH_HIP(pf_quant(b.x, b.xs, b.o, kNH * kHD, M, s));
       r.w[0] = i8p(e, l, R_OP), r.sw[0] = scp(e, l, R_OP);
@@ -811,27 +833,66 @@ int prefill_group(qh_engine* e, const PfBufs& b, int first, int M) {
   return QH_OK;
 }
 
+// Buffers of slot i for groups of G tokens, and with more than one slot its stream and events.
+int prefill_slot(qh_engine* e, int i, int G, bool events) {
+  if (e->pf_cap[i] < G) {
+    if (e->pf[i]) (void)hipFree(e->pf[i]);
+    e->pf[i] = nullptr;
+    e->pf_cap[i] = 0;
+    int cap = 128;
+    while (cap < G) cap *= 2;
+    QH_HIP(hipMalloc(reinterpret_cast<void**>(&e->pf[i]), PfBufs(nullptr, (size_t)cap).bytes));
+    e->pf_cap[i] = cap;
+  }
+  if (e->pf_stream[i] == nullptr) {
+    if (i == 0)
+      e->pf_stream[i] = e->stream;
+    else
+      QH_HIP(hipStreamCreate(&e->pf_stream[i]));
+  }
+  if (events)
+    for (hipEvent_t& ev : e->pf_ev[i])
+      if (ev == nullptr) QH_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  return QH_OK;
+}
+
 // The first n tokens of prompt_dev in groups; *done receives how many ran (0: fed one by one).  A
 // failed launch leaves the state between two tokens' states: decoding is refused until a reset.
 int run_prefill(qh_engine* e, int n, int* done) {
   *done = 0;
   if (n <= 0) return QH_OK;
-  if (e->pf == nullptr) {
-    if (hipMalloc(reinterpret_cast<void**>(&e->pf), PfBufs(nullptr).bytes) != hipSuccess) {
+  const int G = prefill_group_size(n);
+  int slots = n > G ? 2 : 1;
+  for (int i = 0; i < slots; ++i)
+    if (prefill_slot(e, i, G, slots > 1) != QH_OK) {
       (void)hipGetLastError();
-      e->pf = nullptr;
-      e->pf_off = true;
-      return QH_OK;
+      if (i == 0) {
+        e->pf_off = true;
+        return QH_OK;
+      }
+      slots = 1;   // what the first slot needs is there: one group after another
     }
+  const bool events = slots > 1;
+  int st = QH_OK;
+  if (events) {   // the other slots start after the engine stream's earlier work
+    st = hip_status(hipEventRecord(e->pf_ev[0][kLayers], e->stream));
+    for (int i = 1; st == QH_OK && i < slots; ++i) st = hip_status(hipStreamWaitEvent(e->pf_stream[i], e->pf_ev[0][kLayers], 0));
   }
-  const PfBufs b(e->pf);
-  for (int i = 0; i < n; i += kPfGroup) {
-    const int M = n - i < kPfGroup ? n - i : kPfGroup;
-    if (const int st = prefill_group(e, b, i, M); st != QH_OK) {
-      e->broken = true;
-      return st;
-    }
+  const int pos0 = e->host_pos;
+  for (int k = 0, i = 0; st == QH_OK && i < n; ++k, i += G) {
+    const int M = n - i < G ? n - i : G;
+    st = prefill_group(e, k % slots, events && k > 0 ? (k - 1) % slots : -1, events, i, M);
     e->host_pos += M;
+  }
+  for (int i = 1; i < slots; ++i) {   // the engine stream goes on after every slot
+    if (st == QH_OK) st = hip_status(hipEventRecord(e->pf_ev[i][kLayers], e->pf_stream[i]));
+    if (st == QH_OK) st = hip_status(hipStreamWaitEvent(e->stream, e->pf_ev[i][kLayers], 0));
+  }
+  if (st != QH_OK) {
+    for (int i = 0; i < slots; ++i) (void)hipStreamSynchronize(e->pf_stream[i]);
+    e->host_pos = pos0;
+    e->broken = true;
+    return st;
   }
   *done = n;
   return QH_OK;
@@ -847,11 +908,17 @@ void release(qh_engine* e) {
   void* bufs[] = {e->blob, e->rec, e->conv, e->kc, e->vc, e->h, e->convd, e->zb, e->gb, e->o, e->act,
                   e->og, e->qkv, e->pm, e->pl, e->pacc, e->rope, e->logits, e->part_val,
                   e->part_idx, e->ctl, e->prompt_dev, e->out_dev, e->prog[0], e->prog[1], e->arena,
-                  e->abort_dev, e->lanes, e->pf};
+                  e->abort_dev, e->lanes};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (hipEvent_t ev : e->launch_ev)
     if (ev) (void)hipEventDestroy(ev);
+  for (int i = 0; i < kPfSlots; ++i) {
+    if (e->pf[i]) (void)hipFree(e->pf[i]);
+    if (i > 0 && e->pf_stream[i]) (void)hipStreamDestroy(e->pf_stream[i]);
+    for (hipEvent_t ev : e->pf_ev[i])
+      if (ev) (void)hipEventDestroy(ev);
+  }
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
 }

@@ -6,15 +6,18 @@
 // Every value is the token path's, bit for bit, so that a prompt fed through
 // here leaves exactly the state that feeding it token by token leaves:
 //   * W8A8 products are int32 sums, exact in any order: v_mfma_i32_16x16x64_i8.
-//   * W8A16 products follow the C16 order (qh_device.hpp).  v_mfma_f32_16x16x4_f32
-//     computes, for each output, the chain fma(a3,b3,fma(a2,b2,fma(a1,b1,
-//     fma(a0,b0,c)))) with single roundings and denormals kept (compared with
-//     fmaf on 2^20 results), so a lane partial over a 16-element chunk is four
-//     MFMAs from zero; the 64 partials are then added by the same tree.
+//   * W8A16 products follow the C16 order (qh_device.hpp).  The fp32 MFMAs
+//     (v_mfma_f32_16x16x4_f32, v_mfma_f32_32x32x2_f32) compute, for each output,
+//     the chain fma(a1,b1,fma(a0,b0,c)) in increasing k with single roundings and
+//     denormals kept (compared with fmaf on 2^20 results), so a lane partial over
+//     a 16-element chunk is a run of MFMAs from zero; the 64 partials are then
+//     added by the same tree.
 //   * Attention scores (16-lane tree over 16-element chunks) and P.V (a chain in
-//     position order) have the same shape and use the same instruction.
+//     position order) have the same shape and use the same instructions.
 //   * Norms, gates, conv, the delta rule and the softmax repeat the decode
 //     bodies' operations in their order.
+#include <type_traits>
+
 #include "qh_prefill.hpp"
 #include "qh_decode.h"
 #include "qh_stages.hpp"
@@ -25,12 +28,15 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-// lane l's 16-element chunk c of token m, written to the fragments of a K-wide activation
+// 16-element chunk c of token m, written to the fragments of a K-wide activation
 template <int K>
 __device__ __forceinline__ void put_frag_f32(float* x, int m, int c, const float (&v)[16]) {
-  f32x4* p = reinterpret_cast<f32x4*>(x) + ((size_t)(m >> 4) * pf_frags(K) + pf_visit(K, c)) * 64 + (m & 15);
+  f32x4* p = reinterpret_cast<f32x4*>(x + pf_frag_f32(K, m, c, 0));
 #pragma unroll
-  for (int g = 0; g < 4; ++g) *as_global_w(p + 16 * g) = f32x4{v[g], v[4 + g], v[8 + g], v[12 + g]};
+  for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+      *as_global_w(p + 64 * hb + 32 * kk) = f32x4{v[8 * hb + kk], v[8 * hb + 2 + kk], v[8 * hb + 4 + kk], v[8 * hb + 6 + kk]};
 }
 template <int K>
 __device__ __forceinline__ void put_frag_i8(void* x, int m, int c, const uint32_t (&q)[4]) {
@@ -61,6 +67,13 @@ __global__ __launch_bounds__(256) void pf_norm_kernel(const PfNorm a) {
   const int mc = min(m, a.M - 1);
   float xv[16], nw[16];
   load16c(a.nw, lane, nw);
+  float gw[8][16], al = 0.0f, db = 0.0f;   // this wave's gate rows, in flight beside the norm
+  if constexpr (GATES) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) load16c(a.gw + (size_t)(8 * wave + r) * 1024, lane, gw[r]);
+    al = as_global(a.A_log)[(8 * wave + row_of_lane<8>(lane)) & 15];
+    db = as_global(a.dt_bias)[(8 * wave + row_of_lane<8>(lane)) & 15];
+  }
   if (a.emb != nullptr) {
     const int tok = __builtin_amdgcn_readfirstlane(as_global(a.ids)[mc]);
     uint32_t t[4];
@@ -111,231 +124,290 @@ __global__ __launch_bounds__(256) void pf_norm_kernel(const PfNorm a) {
     if (m < a.M) put_frag_f32<1024>(static_cast<float*>(a.x), m, lane, xv);
   }
   if constexpr (GATES) {
-    float gw[8][16];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) load16c(a.gw + (size_t)(8 * wave + r) * 1024, lane, gw[r]);
 #pragma unroll
     for (int k = 0; k < 4; ++k)   // lane-interleaved, as load16c reads
       *as_lds_w(reinterpret_cast<f32x4*>(xl + 1024 * wave + 256 * k + 4 * lane)) =
           f32x4{xv[4 * k], xv[4 * k + 1], xv[4 * k + 2], xv[4 * k + 3]};
     lds_barrier();
+    // lane l ends with row 8 wave + l / 8 of every token and finishes token l % 8 of them
     const int row = 8 * wave + row_of_lane<8>(lane);   // beta rows 0 .. 15, then g
     const int h = row & 15;
-    const float al = as_global(a.A_log)[h], db = as_global(a.dt_bias)[h];
-#pragma unroll 1
+    float y = 0.0f;
+#pragma unroll
     for (int t = 0; t < 4; ++t) {
-      if (m0 + t >= a.M) break;
-      float x[16];
+      float x[16], p[8];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const f32x4 v = *as_lds(reinterpret_cast<const f32x4*>(xl + 1024 * t + 256 * k + 4 * lane));
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[4 * k + e] = v[e];
       }
-      float p[8];
 #pragma unroll
       for (int r = 0; r < 8; ++r) p[r] = dot16_f32(gw[r], x, 0.0f);
-      const float y = reduce8(p, lane);
-      const float val = row < 16 ? dev_sigmoid(y) : dev_expf(-dev_expf(al) * dev_softplus(y + db));
-      if ((lane & 7) == 0) a.gates[((size_t)h * a.M + m0 + t) * 2 + (row < 16 ? 1 : 0)] = val;
+      const float yt = reduce8(p, lane);
+      if ((lane & 7) == t) y = yt;
     }
+    const float val = row < 16 ? dev_sigmoid(y) : dev_expf(-dev_expf(al) * dev_softplus(y + db));
+    const int mt = m0 + (lane & 7);
+    if ((lane & 7) < 4 && mt < a.M) a.gates[((size_t)h * a.M + mt) * 2 + (row < 16 ? 1 : 0)] = val;
   }
 }
 
 // ---------------------------------------------------------------------------
 // Matrix product out[m][n] = sum_k w[n][k] x[m][k].  A workgroup owns TA * 16
-// weight rows, copies them whole (K bytes each) to LDS once, and its four waves
-// multiply them with TB token tiles each; x streams from L2 as fragments, 1 KiB
-// per load instruction.  A (rows of D) = weight rows, B (columns) = tokens, so a
-// lane ends with four consecutive outputs of one token.  A row's 16-byte chunk c
-// sits at chunk c ^ (row & 15): the 16 rows a wave reads at once lie in 16
-// different bank groups.
-// Workgroups with the same rows are a multiple of 8 apart in the grid where the
-// row tiles allow it, so one XCD's L2 serves them all.
+// weight rows, copies them whole (K bytes each) to LDS once, and multiplies them
+// with its token tiles; x streams from L2 as fragments, 1 KiB per load
+// instruction.  A (rows of D) = weight rows, B (columns) = tokens, so a lane ends
+// with four consecutive outputs of one token.  A row's 16-byte chunk c sits at
+// chunk c ^ (row & 15): the 16 rows a wave reads at once lie in 16 different bank
+// groups.  The copy is global -> LDS loads, all in flight at once (through
+// registers, four at a time, it took 12.6 us at K = 3584 where this takes 5).
+//   W8A8   each of the four waves takes its own token tile (an MFMA step is 16
+//          cycles: a tile is too short to share).
+//   W8A16  the four waves split the 64 lanes of the C16 tree, 16 visits each, and
+//          their subtrees meet in LDS: a token tile is 256 MFMAs of 32 cycles per
+//          wave, and a short prompt still fills the chip.
 // ---------------------------------------------------------------------------
-template <int MODE, int K, int TA, int TB, int EPI>
-__global__ __launch_bounds__(256) void pf_gemm_kernel(const PfGemm a) {
-  constexpr int ROWS = 16 * TA, NC = K / 16;
-  __shared__ __attribute__((aligned(16))) int8_t wl[ROWS * K];
+template <int K, int ROWS, int THREADS, class SRC>
+__device__ __forceinline__ void pf_stage_rows(int8_t* wl, SRC src) {
+  constexpr int NC = K / 16;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = lane >> 4, j = lane & 15;
-  const int n0 = (int)blockIdx.x * ROWS;   // first output (PF_SWIGLU: weight) row
-  // the workgroup's rows
+  static_assert((ROWS * NC) % THREADS == 0, "whole passes");
+#pragma unroll
+  for (int i = 0; i < ROWS * NC / THREADS; ++i) {
+    const int u = THREADS * i + 64 * wave, p = u + lane;   // LDS takes a wave's 64 chunks in lane order
+    const int r = p / NC, c = (p % NC) ^ (r & 15);
+    __builtin_amdgcn_global_load_lds(as_global(src(r) + 16 * c), as_lds_w(wl + 16 * u), 16, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+// Outputs 16 ta + 4 g .. + 3 of token m from the scaled-by-activation sums y (PF_SWIGLU: y2 the up
+// row's).  n: the output's column.
+template <int MODE, int EPI>
+__device__ __forceinline__ void pf_epilogue(const PfGemm& a, int si, int m, int n, const f32x4& y, const f32x4& y2) {
+  f32x4 v;
+  if constexpr (EPI == PF_SWIGLU) {
+    const f32x4 sg = *as_global(reinterpret_cast<const f32x4*>(a.sw[0] + n));
+    const f32x4 su = *as_global(reinterpret_cast<const f32x4*>(a.sw[1] + n));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = dev_silu(y[r] * sg[r]) * (y2[r] * su[r]);
+    if constexpr (MODE == M_W8A8) {
+      *as_global_w(reinterpret_cast<f32x4*>(a.out + (size_t)m * a.ld + n)) = v;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) as_global_w(a.out)[pf_frag_f32(QH_INTER, m, n >> 4, (n & 15) + r)] = v[r];
+    }
+  } else {
+    const f32x4 sw = *as_global(reinterpret_cast<const f32x4*>(a.sw[si] + (n - a.row0[si])));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = y[r] * sw[r];
+    f32x4* p = reinterpret_cast<f32x4*>(a.out + (size_t)m * a.ld + n);
+    if constexpr (EPI == PF_INPROJ) {
+      if (si == 1)   // z (the gated norm takes silu(z))
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = dev_silu(v[r]);
+    }
+    if constexpr (EPI == PF_RESID) {
+      const f32x4 h = *as_global(p);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = h[r] + v[r];
+    }
+    *as_global_w(p) = v;
+  }
+}
+
+// the weight segment of output row n0, and the address of the row tile's row r
+template <int EPI>
+__device__ __forceinline__ int pf_seg(const PfGemm& a, int n0) {
   int si = 0;
-  if constexpr (EPI != PF_SWIGLU) {
+  if constexpr (EPI == PF_INPROJ || EPI == PF_STORE) {
 #pragma unroll
     for (int i = 1; i < 3; ++i)
       if (i < a.nseg && n0 >= a.row0[i]) si = i;
   }
-  const int8_t* w0 = a.w[si];
-  const int r0 = n0 - a.row0[si];
-#pragma unroll 4
-  for (int u = threadIdx.x; u < ROWS * NC; u += 256) {
-    const int r = u / NC, c = u % NC;
-    const int8_t* src;
-    if constexpr (EPI == PF_SWIGLU) {   // 16-row blocks alternate gate, up
-      const int t = r >> 4;
-      src = ((t & 1) ? a.w[1] : a.w[0]) + (size_t)(n0 / 2 + (t >> 1) * 16 + (r & 15)) * K + 16 * c;
-    } else {
-      src = w0 + (size_t)(r0 + r) * K + 16 * c;
-    }
-    const u32x4 v = *as_global(reinterpret_cast<const u32x4*>(src));
-    *as_lds_w(reinterpret_cast<u32x4*>(wl + r * K + 16 * (c ^ (r & 15)))) = v;
+  return si;
+}
+template <int K, int EPI>
+__device__ __forceinline__ const int8_t* pf_row(const PfGemm& a, int si, int n0, int r) {
+  if constexpr (EPI == PF_SWIGLU) {   // 16-row blocks alternate gate, up
+    const int t = r >> 4;
+    return ((t & 1) ? a.w[1] : a.w[0]) + (size_t)(n0 / 2 + (t >> 1) * 16 + (r & 15)) * K;
+  } else {
+    return a.w[si] + (size_t)(n0 - a.row0[si] + r) * K;
   }
-  __syncthreads();
+}
+
+template <int K, int TA, int EPI>
+__global__ __launch_bounds__(256) void pf_gemm_i8_kernel(const PfGemm a, int tpw) {
+  constexpr int ROWS = 16 * TA, NS = K / 64;
+  __shared__ __attribute__((aligned(16))) int8_t wl[ROWS * K];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, j = lane & 15;
+  const int n0 = (int)blockIdx.x * ROWS;   // first output (PF_SWIGLU: weight) row
+  const int si = pf_seg<EPI>(a, n0);
   const int ntile = (a.M + 15) >> 4;
-  const int tt0 = ((int)blockIdx.y * 4 + wave) * TB;
-  if (tt0 >= ntile) return;   // no barrier follows
-  f32x4 y[TA][TB];
-  if constexpr (MODE == M_W8A8) {
-    i32x4 acc[TA][TB];
+  const int t0 = (int)blockIdx.y * tpw, t1 = min(t0 + tpw, ntile);
+  constexpr int PF = NS % 8 == 0 ? 8 : 7;   // steps of x in flight
+  static_assert(NS % PF == 0, "steps");
+  const i32x4* xb0 = reinterpret_cast<const i32x4*>(a.x) + lane;
+  i32x4 xb[PF];
+  int tt = t0 + wave;
+  {   // the first tile's x is in flight beside the rows
+    const i32x4* xp = xb0 + (size_t)min(tt, ntile - 1) * NS * 64;
 #pragma unroll
-    for (int ta = 0; ta < TA; ++ta)
+    for (int p = 0; p < PF; ++p) xb[p] = *as_global(xp + 64 * p);
+  }
+  pf_stage_rows<K, ROWS, 256>(wl, [&](int r) { return pf_row<K, EPI>(a, si, n0, r); });
+  for (; tt < t1; tt += 4) {
+    const i32x4* xp = xb0 + (size_t)tt * NS * 64;
+    const i32x4* xn = xb0 + (size_t)min(tt + 4, ntile - 1) * NS * 64;   // the next tile's
+    i32x4 acc[TA];
 #pragma unroll
-      for (int tb = 0; tb < TB; ++tb) acc[ta][tb] = i32x4{0, 0, 0, 0};
-    const i32x4* xp[TB];
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb)
-      xp[tb] = reinterpret_cast<const i32x4*>(a.x) + (size_t)min(tt0 + tb, ntile - 1) * (K / 64) * 64 + lane;
-    constexpr int PF = 4;   // steps of x in flight
-    static_assert((K / 64) % PF == 0, "steps");
-    i32x4 xb[PF][TB];
-#pragma unroll
-    for (int p = 0; p < PF; ++p)
-#pragma unroll
-      for (int tb = 0; tb < TB; ++tb) xb[p][tb] = *as_global(xp[tb] + 64 * p);
+    for (int ta = 0; ta < TA; ++ta) acc[ta] = i32x4{0, 0, 0, 0};
 #pragma unroll 1
-    for (int s0 = 0; s0 < K / 64; s0 += PF) {
+    for (int s0 = 0; s0 < NS; s0 += PF) {
+      const i32x4* xq = s0 + PF < NS ? xp + 64 * (s0 + PF) : xn;
 #pragma unroll
       for (int p = 0; p < PF; ++p) {
         const int s = s0 + p;
-        i32x4 wa[TA];
+        const i32x4 b = xb[p];
+        xb[p] = *as_global(xq + 64 * p);
 #pragma unroll
-        for (int ta = 0; ta < TA; ++ta)
-          wa[ta] = *as_lds(reinterpret_cast<const i32x4*>(wl + (16 * ta + j) * K + 16 * ((4 * s + g) ^ j)));
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb) {
-          const i32x4 b = xb[p][tb];
-          xb[p][tb] = *as_global(xp[tb] + 64 * min(s + PF, K / 64 - 1));
-#pragma unroll
-          for (int ta = 0; ta < TA; ++ta)
-            acc[ta][tb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[ta], b, acc[ta][tb], 0, 0, 0);
+        for (int ta = 0; ta < TA; ++ta) {
+          const i32x4 wa = *as_lds(reinterpret_cast<const i32x4*>(wl + (16 * ta + j) * K + 16 * ((4 * s + g) ^ j)));
+          acc[ta] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa, b, acc[ta], 0, 0, 0);
         }
       }
     }
-#pragma unroll
-    for (int tb = 0; tb < TB; ++tb) {
-      const float xs = as_global(a.xs)[min(16 * (tt0 + tb) + j, a.M - 1)];
+    const int m = 16 * tt + j;
+    if (m < a.M) {
+      const float xs = as_global(a.xs)[m];
+      f32x4 y[TA];
 #pragma unroll
       for (int ta = 0; ta < TA; ++ta)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) y[ta][tb][r] = (float)acc[ta][tb][r] * xs;
-    }
-  } else {
-    static_assert(TB == 1, "one token tile per wave");
-    constexpr int NCH = pf_nch(K);
-    const f32x4* xp = reinterpret_cast<const f32x4*>(a.x) + (size_t)tt0 * pf_frags(K) * 64 + lane;
-    f32x4 t0[TA], t1[TA], t2[TA];
-    // Eight lanes' partials (visits 8 w8 .. 8 w8 + 7) and their three tree levels at a time; a
-    // visit's x is replaced by the visit's eight later as soon as it is read.
-    f32x4 xb[8 * NCH];
-    auto xload = [&](int w8, int i) { return *as_global(xp + 64 * (8 * NCH * min(w8, 7) + i)); };
+        for (int r = 0; r < 4; ++r) y[ta][r] = (float)acc[ta][r] * xs;
+      if constexpr (EPI == PF_SWIGLU) {
 #pragma unroll
-    for (int i = 0; i < 8 * NCH; ++i) xb[i] = xload(0, i);
-#pragma unroll 1
-    for (int w8 = 0; w8 < 8; ++w8) {
-      // lane of the tree: bit-reversed visit; its low three bits come from w8
-      const int lb = ((w8 >> 2) & 1) | (w8 & 2) | ((w8 & 1) << 2);
-      f32x4 part[8][TA];   // (folded as soon as a pair is complete; at most four are live)
+        for (int ta = 0; ta < TA; ta += 2)
+          pf_epilogue<M_W8A8, EPI>(a, si, m, n0 / 2 + (ta >> 1) * 16 + 4 * g, y[ta], y[ta + 1]);
+      } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int l = lb + 8 * (((i >> 2) & 1) | (i & 2) | ((i & 1) << 2));
-#pragma unroll
-        for (int ta = 0; ta < TA; ++ta) part[i][ta] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int jj = 0; jj < NCH; ++jj) {
-          if (64 * jj + 32 >= NC && (i & 1)) continue;   // chunk past K: only lanes below 32 hold it (odd visits: lanes 32 ..)
-          const int c = l + 64 * jj;
-          const f32x4 b = xb[i * NCH + jj];
-          xb[i * NCH + jj] = xload(w8 + 1, i * NCH + jj);
-#pragma unroll
-          for (int ta = 0; ta < TA; ++ta) {
-            const u32x4 wv = *as_lds(reinterpret_cast<const u32x4*>(wl + (16 * ta + j) * K + 16 * (c ^ j)));
-            // elements g, 4 + g, 8 + g, 12 + g: byte g of the four dwords
-            const float f0 = (float)(int)(int8_t)(wv[0] >> (8 * g)), f1 = (float)(int)(int8_t)(wv[1] >> (8 * g)),
-                        f2 = (float)(int)(int8_t)(wv[2] >> (8 * g)), f3 = (float)(int)(int8_t)(wv[3] >> (8 * g));
-            part[i][ta] = __builtin_amdgcn_mfma_f32_16x16x4f32(f0, b[0], part[i][ta], 0, 0, 0);
-            part[i][ta] = __builtin_amdgcn_mfma_f32_16x16x4f32(f1, b[1], part[i][ta], 0, 0, 0);
-            part[i][ta] = __builtin_amdgcn_mfma_f32_16x16x4f32(f2, b[2], part[i][ta], 0, 0, 0);
-            part[i][ta] = __builtin_amdgcn_mfma_f32_16x16x4f32(f3, b[3], part[i][ta], 0, 0, 0);
-          }
-        }
-        if (i & 1) {   // the tree's levels at offsets 32, 16, 8
-#pragma unroll
-          for (int ta = 0; ta < TA; ++ta) {
-            part[i - 1][ta] = part[i - 1][ta] + part[i][ta];
-            if ((i & 3) == 3) part[i - 3][ta] = part[i - 3][ta] + part[i - 1][ta];
-            if (i == 7) part[0][ta] = part[0][ta] + part[4][ta];
-          }
-        }
-      }
-      // offsets 4, 2, 1: a binary counter over the eight groups of eight
-#pragma unroll
-      for (int ta = 0; ta < TA; ++ta) {
-        f32x4 r = part[0][ta];
-        if (w8 & 1) r = t0[ta] + r;
-        else t0[ta] = r;
-        if ((w8 & 3) == 3) r = t1[ta] + r;
-        else if (w8 & 1) t1[ta] = r;
-        if (w8 == 7) r = t2[ta] + r;
-        else if (w8 == 3) t2[ta] = r;
-        y[ta][0] = r;
+        for (int ta = 0; ta < TA; ++ta) pf_epilogue<M_W8A8, EPI>(a, si, m, n0 + 16 * ta + 4 * g, y[ta], y[ta]);
       }
     }
   }
-  // ---- epilogue: token m, outputs 16 ta + 4 g .. + 3 of the row tile
+}
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// RT row tiles of 32 rows; each is shared by KS waves, which take 64 / KS visits each.
+template <int K, int RT, int KS, int EPI>
+__global__ __launch_bounds__(64 * RT * KS, 2) void pf_gemm_f32_kernel(const PfGemm a, int tpw) {
+  constexpr int ROWS = 32 * RT, NC = K / 16, NCH = pf_nch(K), NW = RT * KS, NV = 64 / KS;
+  constexpr int LG = NV == 32 ? 5 : NV == 16 ? 4 : 3;   // tree levels inside a wave
+  static_assert(NV == 1 << LG, "visits per wave");
+  __shared__ __attribute__((aligned(16))) int8_t wl[ROWS * K];
+  __shared__ __attribute__((aligned(16))) float red[NW * 4 * 256];   // subtree sums [wave][group of 4 rows][lane]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ks = wave % KS, rt = wave / KS;
+  const int kk = lane >> 5, j = lane & 31;
+  const int n0 = (int)blockIdx.x * ROWS;
+  const int si = pf_seg<EPI>(a, n0);
+  const int ntile = (a.M + 31) >> 5;
+  const int t0 = (int)blockIdx.y * tpw, t1 = min(t0 + tpw, ntile);
+  constexpr int NX = NV * NCH, PF = 4;   // steps (chunks) of a wave and tile; x of PF steps in flight
+  const f32x4* xw = reinterpret_cast<const f32x4*>(a.x) + 128 * NX * ks + lane;
+  f32x4 xb[PF][2];
 #pragma unroll
-  for (int tb = 0; tb < TB; ++tb) {
-    const int m = 16 * (tt0 + tb) + j;
-    if (tt0 + tb >= ntile || m >= a.M) continue;
-    if constexpr (EPI == PF_SWIGLU) {
+  for (int p = 0; p < PF; ++p)
 #pragma unroll
-      for (int ta = 0; ta < TA; ta += 2) {
-        const int n = n0 / 2 + (ta >> 1) * 16 + 4 * g;
-        const f32x4 sg = *as_global(reinterpret_cast<const f32x4*>(a.sw[0] + n));
-        const f32x4 su = *as_global(reinterpret_cast<const f32x4*>(a.sw[1] + n));
-        f32x4 v;
+    for (int hb = 0; hb < 2; ++hb) xb[p][hb] = *as_global(xw + (size_t)t0 * pf_frags(K) * 128 + 128 * p + 64 * hb);
+  pf_stage_rows<K, ROWS, 64 * NW>(wl, [&](int r) { return pf_row<K, EPI>(a, si, n0, r); });
+  // lane of the tree = the visit's six bits reversed: visits NV ks + i lie at lanes (ks reversed) + KS * (i reversed)
+  const int lw = pf_bitrev6(ks * NV);
+  // step f = visit f / NCH, chunk f % NCH of its lane; past K (the tree's upper 32 lanes, the odd
+  // visits, have one chunk less at K = 3584) there is no step
+  auto live = [](int f) constexpr { return !(64 * (f % NCH) + 32 >= NC && ((f / NCH) & 1)); };
+  auto next = [&](int f) constexpr {   // the next step; the last one is followed by the next tile's first
+    do f = f + 1 == NX ? 0 : f + 1;
+    while (!live(f));
+    return f;
+  };
+  auto wread = [&](int f) {   // the rows' chunk of step f
+    const int l = lw + pf_bitrev6(f / NCH);
+    return *as_lds(reinterpret_cast<const u32x4*>(wl + (32 * rt + j) * K + 16 * ((l + 64 * (f % NCH)) ^ (j & 15))));
+  };
+  u32x4 wv = wread(0);
+  for (int tt = t0; tt < t1; ++tt) {
+    const f32x4* xp = xw + (size_t)tt * pf_frags(K) * 128;
+    const f32x4* xn = xw + (size_t)min(tt + 1, t1 - 1) * pf_frags(K) * 128;   // the next tile's
+    f32x16 st[LG], part;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = dev_silu(y[ta][tb][r] * sg[r]) * (y[ta + 1][tb][r] * su[r]);
-        if constexpr (MODE == M_W8A8) {
-          *as_global_w(reinterpret_cast<f32x4*>(a.out + (size_t)m * a.ld + n)) = v;
-        } else {   // element 4 g + r of chunk n / 16: fragment lane group r, position g
-          const int c = n >> 4;
-          float* p = a.out + (((size_t)(m >> 4) * pf_frags(QH_INTER) + pf_visit(QH_INTER, c)) * 64 + (m & 15)) * 4 + g;
+    for (int f = 0; f < NX; ++f) {
+      const int i = f / NCH;
+      if (f % NCH == 0) part = f32x16{};
+      f32x4 b[2];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) as_global_w(p)[64 * r] = v[r];
+      for (int hb = 0; hb < 2; ++hb) {
+        b[hb] = xb[f % PF][hb];
+        xb[f % PF][hb] = *as_global(f + PF < NX ? xp + 128 * (f + PF) + 64 * hb : xn + 128 * (f + PF - NX) + 64 * hb);
+      }
+      if (live(f)) {
+        float wf[8];   // elements 2 e + kk
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const uint32_t t = wv[d] >> (8 * kk);
+          wf[2 * d] = (float)(int)(int8_t)t;
+          wf[2 * d + 1] = (float)(int)(int8_t)(t >> 16);
+        }
+        wv = wread(next(f));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[e], b[e >> 2][e & 3], part, 0, 0, 0);
+      }
+      if (f % NCH != NCH - 1) continue;
+      // the tree's first LG levels (offsets 32, 16, ...): a binary counter over the visits
+#pragma unroll
+      for (int v = 0; v < LG; ++v) {
+        const int bits = (1 << v) - 1;
+        if ((i & bits) != bits) break;
+        if ((i >> v) & 1)
+          part = st[v] + part;
+        else {
+          st[v] = part;
+          break;
         }
       }
+    }
+    // the remaining levels: the waves' subtrees of each row tile
+    lds_barrier();   // the previous sums have been read
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *as_lds_w(reinterpret_cast<f32x4*>(red + (wave * 4 + q) * 256 + 4 * lane)) =
+          f32x4{part[4 * q], part[4 * q + 1], part[4 * q + 2], part[4 * q + 3]};
+    lds_barrier();
+    auto total = [&](int r, int q) {   // rows 8 q + 4 kk .. + 3 of row tile r
+      f32x4 s[KS];
+#pragma unroll
+      for (int w = 0; w < KS; ++w) s[w] = *as_lds(reinterpret_cast<const f32x4*>(red + ((r * KS + w) * 4 + q) * 256 + 4 * lane));
+#pragma unroll
+      for (int d = 1; d < KS; d *= 2)
+#pragma unroll
+        for (int w = 0; w < KS; w += 2 * d) s[w] = s[w] + s[w + d];
+      return s[0];
+    };
+    const int m = 32 * tt + j;
+    if constexpr (EPI == PF_SWIGLU) {   // gate rows 16 .. apart from their up rows
+      for (int u = wave; u < 2 * RT; u += NW) {
+        const f32x4 y = total(u >> 1, u & 1), y2 = total(u >> 1, (u & 1) + 2);
+        if (m < a.M) pf_epilogue<M_W8A16, EPI>(a, si, m, n0 / 2 + 8 * u + 4 * kk, y, y2);
+      }
     } else {
-#pragma unroll
-      for (int ta = 0; ta < TA; ++ta) {
-        const int n = n0 + 16 * ta + 4 * g;
-        const f32x4 sw = *as_global(reinterpret_cast<const f32x4*>(a.sw[si] + (n - a.row0[si])));
-        f32x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = y[ta][tb][r] * sw[r];
-        f32x4* p = reinterpret_cast<f32x4*>(a.out + (size_t)m * a.ld + n);
-        if constexpr (EPI == PF_INPROJ) {
-          if (si == 1)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = dev_silu(v[r]);
-        }
-        if constexpr (EPI == PF_RESID) {
-          const f32x4 h = *as_global(p);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = h[r] + v[r];
-        }
-        *as_global_w(p) = v;
+      for (int u = wave; u < 4 * RT; u += NW) {
+        const f32x4 y = total(u >> 2, u & 3);
+        if (m < a.M) pf_epilogue<M_W8A16, EPI>(a, si, m, n0 + 8 * u + 4 * kk, y, y);
       }
     }
   }
@@ -343,51 +415,64 @@ __global__ __launch_bounds__(256) void pf_gemm_kernel(const PfGemm a) {
 
 // ---------------------------------------------------------------------------
 // Short conv + SiLU of the raw qkv rows, then the l2norm of q and k (and q's
-// 1 / sqrt(128)): thread c takes channels 16 c .. 16 c + 15 (one k-group of a
-// head) for kConvTok tokens in a row, its window in registers.  q and k of
-// (head, token) go to 256 floats: element e of k-group kg of q at
-// (e / 4) * 32 + 4 kg + e % 4, k 128 further (the order the scan's lanes read).
+// 1 / sqrt(128)), kConvTok tokens per workgroup.  The convolution is elementwise:
+// thread t takes channel quads t, t + 384, ... so that every load of a wave is
+// consecutive memory, and the results meet in LDS, from which thread c takes
+// channels 16 c .. 16 c + 15 (one k-group of a head) for the norm.  (With 16
+// channels per thread from the start each tap load touched 64 cache lines: 27 us
+// at 512 tokens.)  q and k of (head, token) go to 256 floats in the order the
+// scan reads them: elements 8 e2 + 4 qd .. + 3 of q (e2 = half of a k-group) at
+// 64 qd + 4 e2, k 128 further.
 // ---------------------------------------------------------------------------
-constexpr int kConvTok = 4;
+constexpr int kConvTok = 2;
 __global__ __launch_bounds__(384) void pf_conv_kernel(const PfConv a) {
-  const int c = threadIdx.x, ch = 16 * c;
-  const int m0 = (int)blockIdx.x * kConvTok;
-  float taps[16][4];
+  __shared__ __attribute__((aligned(16))) float xl[kConvTok * QH_CONV_DIM];
+  const int t = threadIdx.x, m0 = (int)blockIdx.x * kConvTok;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const f32x4 t = *as_global(reinterpret_cast<const f32x4*>(a.taps + (size_t)(ch + e) * 4));
+  for (int u = 0; u < 4; ++u) {
+    const int ch = 4 * (t + 384 * u);
+    f32x4 in[3 + kConvTok], tap[4];   // rows m0 - 3 ..; taps of the four channels
 #pragma unroll
-    for (int k = 0; k < 4; ++k) taps[e][k] = t[k];
-  }
-  float w1[16], w2[16], w3[16];   // the window's older inputs, oldest first
-  auto row = [&](int m, float (&v)[16]) {   // input m of the group; before it, the state's columns 1 .. 3
-    if (m >= 0) {
-      load16g(a.y + (size_t)m * 8192 + ch, v);
+    for (int e = 0; e < 4; ++e) tap[e] = *as_global(reinterpret_cast<const f32x4*>(a.taps + (size_t)(ch + e) * 4));
+    if (m0 < 3) {   // rows before the group: columns 1 .. 3 of the state (row -i in column 4 - i)
+      f32x4 st[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[e] = *as_global(reinterpret_cast<const f32x4*>(a.state + (size_t)(ch + e) * 4));
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int m = m0 - 3 + i;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) in[i][e] = m == -3 ? st[e][1] : m == -2 ? st[e][2] : st[e][3];
+        if (m >= 0) in[i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)m * 8192 + ch));
+      }
     } else {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) v[e] = as_global(a.state)[(size_t)(ch + e) * 4 + 4 + m];
+      for (int i = 0; i < 3; ++i) in[i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)(m0 - 3 + i) * 8192 + ch));
     }
-  };
-  row(m0 - 3, w1);
-  row(m0 - 2, w2);
-  row(m0 - 1, w3);
-  const int part = c >> 7, h = (c & 127) >> 3, kg = c & 7;   // q, k or v; head; k-group
-#pragma unroll 1
-  for (int m = m0; m < min(m0 + kConvTok, a.M); ++m) {
-    float y[16], x[16];
-    row(m, y);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      float acc = 0.0f;
-      acc = acc + w1[e] * taps[e][0];
-      acc = acc + w2[e] * taps[e][1];
-      acc = acc + w3[e] * taps[e][2];
-      acc = acc + y[e] * taps[e][3];
-      x[e] = dev_silu(acc);
-      w1[e] = w2[e];
-      w2[e] = w3[e];
-      w3[e] = y[e];
+    for (int i = 0; i < kConvTok; ++i)
+      in[3 + i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)min(m0 + i, a.M - 1) * 8192 + ch));
+#pragma unroll
+    for (int k = 0; k < kConvTok; ++k) {
+      f32x4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float acc = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = acc + in[k + i][e] * tap[e][i];
+        x[e] = dev_silu(acc);
+      }
+      *as_lds_w(reinterpret_cast<f32x4*>(xl + k * QH_CONV_DIM + ch)) = x;
     }
+  }
+  lds_barrier();
+  const int c = t, part = c >> 7, h = (c & 127) >> 3, kg = c & 7;   // q, k or v; head; k-group
+#pragma unroll 1
+  for (int k = 0; k < kConvTok; ++k) {
+    const int m = m0 + k;
+    if (m >= a.M) break;
+    float x[16];
+    load16l(xl + k * QH_CONV_DIM + 16 * c, x);
     if (part < 2) {   // deltanet.hpp:134,166-169 (whole waves: c / 128 is wave-uniform)
       float ss = dot16_f32(x, x, 0.0f);
       ss = xor_sum<8>(ss);
@@ -399,101 +484,181 @@ __global__ __launch_bounds__(384) void pf_conv_kernel(const PfConv a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) x[e] = x[e] * sc;
       }
-      float* p = a.qk + ((size_t)h * a.M + m) * 256 + 128 * part + 4 * kg;
+      float* p = a.qk + ((size_t)h * a.M + m) * 256 + 128 * part + 8 * kg;
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        *as_global_w(reinterpret_cast<f32x4*>(p + 32 * k)) = f32x4{x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]};
+      for (int d = 0; d < 4; ++d)   // half d / 2, quad d % 2
+        *as_global_w(reinterpret_cast<f32x4*>(p + 64 * (d & 1) + 4 * (d >> 1))) =
+            f32x4{x[4 * d], x[4 * d + 1], x[4 * d + 2], x[4 * d + 3]};
     } else {
       float* p = a.v + ((size_t)h * a.M + m) * 128 + 16 * kg;
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        *as_global_w(reinterpret_cast<f32x4*>(p + 4 * k)) = f32x4{x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]};
+      for (int d = 0; d < 4; ++d)
+        *as_global_w(reinterpret_cast<f32x4*>(p + 4 * d)) = f32x4{x[4 * d], x[4 * d + 1], x[4 * d + 2], x[4 * d + 3]};
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// The delta rule over the group's tokens in order (deltanet_body's operations):
-// one wave per workgroup and 8 columns of one head, 256 workgroups, so every
-// wave has a CU's vector memory and LDS paths to itself; the wave's 128 x 8
-// slice of S stays in registers for the whole group.  Bound by its own serial
-// chain of about 125 vector instructions per token; q, k, v and the gates of the
-// next eight tokens are in flight while eight are computed.
+// The delta rule over the group's tokens in order (deltanet_body's operations).
+// It is bound by the serial chain of one token after another: p = sum_k s k over
+// 16 elements in sequence and a tree of eight, delta, the update.  To shorten
+// what one wave issues per token:
+//   * a 16-element chain is shared by two lanes, eight elements each: the even
+//     lane's partial sum passes to the odd lane, which continues it, and the
+//     multiplies and updates beside the chain halve;
+//   * the output q^T S runs on a second wave with its own copy of the slice, one
+//     block of eight tokens behind: the first wave (A) computes delta and leaves
+//     it in LDS, the second (B) repeats decay and update and forms the output.
+// A workgroup holds 8 columns of one head on four waves (A and B for columns
+// 0 .. 3, A and B for 4 .. 7): 256 workgroups, one wave per SIMD.  One barrier
+// per eight tokens.  A token took 835 cycles with the whole column group's chain
+// on one wave.
 // ---------------------------------------------------------------------------
 constexpr int kScanTok = 8;
-__global__ __launch_bounds__(64, 1) void pf_scan_kernel(const PfScan a) {
-  __shared__ __attribute__((aligned(16))) float qkl[2][kScanTok * 256];
-  __shared__ __attribute__((aligned(16))) float vl[2][64];
-  const int lane = threadIdx.x, kg = lane & 7, vc = lane >> 3;
-  const int h = (int)blockIdx.x >> 4, v = ((int)blockIdx.x & 15) * 8 + vc;
-  const int M = a.M;
-  float* Sh = a.S + (size_t)h * 128 * 128;
-  float s[16];
+struct ScanBlock {   // eight tokens of q, k (256 floats each, see pf_conv_kernel), v [token][8 columns], gates
+  float qk[kScanTok * 256];
+  float v[kScanTok * 8];
+  float g[kScanTok * 2];
+};
+// a value of the even lane of each pair in both lanes / of the odd lane
+__device__ __forceinline__ float pair_even(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xA0, 0xF, 0xF, false));   // quad_perm [0,0,2,2]
+}
+__device__ __forceinline__ float pair_odd(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xF5, 0xF, 0xF, false));   // quad_perm [1,1,3,3]
+}
+// sum over i of a[i] b[i] over the pair's 16 elements in order, then over the eight k-groups: valid in odd lanes
+__device__ __forceinline__ float scan_dot(const float (&a)[8], const float (&b)[8]) {
+  float t[8];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) s[i] = as_global(Sh)[(kg * 16 + i) * 128 + v];
+  for (int i = 0; i < 8; ++i) t[i] = a[i] * b[i];
+  float p = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) p = p + t[i];
+  p = pair_even(p);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) p = p + t[i];
+  p = p + xor_perm<8>(p);   // k-groups 4, 2, 1 apart
+  p = p + xor_perm<4>(p);
+  p = p + xor_perm<2>(p);
+  return p;
+}
+__global__ __launch_bounds__(256, 1) void pf_scan_kernel(const PfScan a) {
+  __shared__ __attribute__((aligned(16))) ScanBlock blk[3];   // being filled, A's, B's
+  __shared__ float dl[2][2 * 4 * kScanTok];                   // delta [A wave][token][column]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kh = lane & 15, kg = kh >> 1, vc = lane >> 4;     // half k-group, k-group, column of the wave
+  const int half = wave & 1;                                  // columns 4 half ..
+  const bool isA = wave < 2;
+  const int h = (int)blockIdx.x >> 4, v0 = ((int)blockIdx.x & 15) * 8, v = v0 + 4 * half + vc;
+  const int M = a.M, nb = (M + kScanTok - 1) / kScanTok;
+  float* Sh = a.S + (size_t)h * 128 * 128;
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s[i] = as_global(Sh)[(kh * 8 + i) * 128 + v];
   const float* qk = a.qk + (size_t)h * M * 256;
   const float* vp = a.v + (size_t)h * M * 128;
   const float* gp = a.gates + (size_t)h * M * 2;
-  f32x4 nq[kScanTok];
-  float nv, ng;   // lane: v of token lane & 7, column lane >> 3; gate lane & 1 of token (lane >> 1) & 7
-  auto fetch = [&](int m0) {
-#pragma unroll
-    for (int t = 0; t < kScanTok; ++t)
-      nq[t] = *as_global(reinterpret_cast<const f32x4*>(qk + (size_t)min(m0 + t, M - 1) * 256 + 4 * lane));
-    nv = as_global(vp)[(size_t)min(m0 + kg, M - 1) * 128 + v];
-    ng = as_global(gp)[(size_t)min(m0 + ((lane >> 1) & 7), M - 1) * 2 + (lane & 1)];
+  // a block's loads: every thread 32 bytes of q, k; wave 0 v, wave 1 the gates
+  f32x4 n0, n1;
+  float nx = 0.0f;
+  auto fetch = [&](int b) {
+    const int m0 = b * kScanTok, t = threadIdx.x;
+    const float* p = qk + (size_t)min(m0 + (t >> 5), M - 1) * 256 + 8 * (t & 31);
+    n0 = *as_global(reinterpret_cast<const f32x4*>(p));
+    n1 = *as_global(reinterpret_cast<const f32x4*>(p + 4));
+    if (wave == 0) nx = as_global(vp)[(size_t)min(m0 + (lane >> 3), M - 1) * 128 + v0 + (lane & 7)];
+    if (wave == 1) nx = as_global(gp)[(size_t)min(m0 + ((lane >> 1) & 7), M - 1) * 2 + (lane & 1)];
   };
-  fetch(0);
-  int buf = 0;
-#pragma unroll 1
-  for (int m0 = 0; m0 < M; m0 += kScanTok, buf ^= 1) {
+  auto put = [&](int b) {
+    ScanBlock& k = blk[b % 3];
+    *as_lds_w(reinterpret_cast<f32x4*>(k.qk + 8 * threadIdx.x)) = n0;
+    *as_lds_w(reinterpret_cast<f32x4*>(k.qk + 8 * threadIdx.x + 4)) = n1;
+    if (wave == 0) as_lds_w(k.v)[lane] = nx;
+    if (wave == 1 && lane < 16) as_lds_w(k.g)[lane] = nx;
+  };
+  auto ld8 = [&](const float* p, float (&o)[8]) {   // this lane's 8 elements of q (k: 128 further)
+    const f32x4 x = *as_lds(reinterpret_cast<const f32x4*>(p + 4 * kh));
+    const f32x4 y = *as_lds(reinterpret_cast<const f32x4*>(p + 64 + 4 * kh));
 #pragma unroll
-    for (int t = 0; t < kScanTok; ++t) *as_lds_w(reinterpret_cast<f32x4*>(&qkl[buf][256 * t + 4 * lane])) = nq[t];
-    as_lds_w(vl[buf])[lane] = nv;
-    const float cg = ng;
-    lds_barrier();   // one wave: orders its own LDS writes and reads
-    if (m0 + kScanTok < M) fetch(m0 + kScanTok);
-    const int n = min(kScanTok, M - m0);
+    for (int e = 0; e < 4; ++e) {
+      o[e] = x[e];
+      o[4 + e] = y[e];
+    }
+  };
+  // n tokens of block b (FULL: all eight, straight-line)
+  auto runA = [&](int b, auto full, int n) {
+    const ScanBlock& B = blk[b % 3];
+    float* d_out = dl[b & 1] + 32 * half;
+    const float cg = as_lds(B.g)[lane & 15];
+#pragma unroll
+    for (int t = 0; t < kScanTok; ++t) {
+      if (!decltype(full)::value && t >= n) break;
+      float k[8];
+      ld8(B.qk + 256 * t + 128, k);
+      const float vt = as_lds(B.v)[8 * t + 4 * half + vc];
+      const float gexp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t));
+      const float beta = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t + 1));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] = s[i] * gexp;
+      const float d = pair_odd((vt - scan_dot(s, k)) * beta);
+      if (kh == 0) as_lds_w(d_out)[4 * t + vc] = d;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] = s[i] + k[i] * d;
+    }
+  };
+  auto runB = [&](int b, auto full, int n) {
+    const ScanBlock& B = blk[b % 3];
+    const float* d_in = dl[b & 1] + 32 * half;
+    const float cg = as_lds(B.g)[lane & 15];
     float ov = 0.0f;
 #pragma unroll
     for (int t = 0; t < kScanTok; ++t) {
-      if (t < n) {
-        float q[16], k[16];
+      if (!decltype(full)::value && t >= n) break;
+      float k[8], q[8];
+      ld8(B.qk + 256 * t + 128, k);
+      ld8(B.qk + 256 * t, q);
+      const float d = as_lds(d_in)[4 * t + vc];
+      const float gexp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t));
 #pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-          const f32x4 x = *as_lds(reinterpret_cast<const f32x4*>(&qkl[buf][256 * t + 32 * qd + 4 * kg]));
-          const f32x4 z = *as_lds(reinterpret_cast<const f32x4*>(&qkl[buf][256 * t + 128 + 32 * qd + 4 * kg]));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            q[4 * qd + e] = x[e];
-            k[4 * qd + e] = z[e];
-          }
-        }
-        const float vt = as_lds(vl[buf])[8 * vc + t];
-        const float gexp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t));
-        const float beta = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t + 1));
-        float p = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          s[i] = s[i] * gexp;
-          p = p + s[i] * k[i];
-        }
-        p = xor_sum<8>(p);
-        const float d = (vt - p) * beta;
-        p = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          s[i] = s[i] + k[i] * d;
-          p = p + s[i] * q[i];
-        }
-        p = xor_sum<8>(p);
-        if (kg == t) ov = p;
+      for (int i = 0; i < 8; ++i) {
+        s[i] = s[i] * gexp;
+        s[i] = s[i] + k[i] * d;
       }
+      const float p = scan_dot(s, q);
+      if (kg == t) ov = p;
     }
-    if (kg < n) as_global_w(a.o)[(size_t)(m0 + kg) * 2048 + h * 128 + v] = ov;
+    if ((lane & 1) && kg < n) as_global_w(a.o)[(size_t)(b * kScanTok + kg) * 2048 + h * 128 + v] = ov;
+  };
+  using T = std::integral_constant<bool, true>;
+  using F = std::integral_constant<bool, false>;
+  fetch(0);
+  put(0);
+  if (nb > 1) fetch(1);
+  lds_barrier();
+#pragma unroll 1
+  for (int b = 0; b <= nb; ++b) {   // A on block b, B on block b - 1; block b + 1 goes to LDS
+    if (b + 1 < nb) {
+      put(b + 1);
+      if (b + 2 < nb) fetch(b + 2);
+    }
+    if (isA) {
+      if (b < nb) {
+        const int n = min(kScanTok, M - b * kScanTok);
+        if (n == kScanTok) runA(b, T{}, n);
+        else runA(b, F{}, n);
+      }
+    } else if (b > 0) {
+      const int n = min(kScanTok, M - (b - 1) * kScanTok);
+      if (n == kScanTok) runB(b - 1, T{}, n);
+      else runB(b - 1, F{}, n);
+    }
+    lds_barrier();
   }
+  if (isA) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) as_global_w(Sh)[(kg * 16 + i) * 128 + v] = s[i];
+    for (int i = 0; i < 8; ++i) as_global_w(Sh)[(kh * 8 + i) * 128 + v] = s[i];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -841,10 +1006,9 @@ __global__ __launch_bounds__(256, 1) void pf_attn_kernel(const PfAttn a) {
         if constexpr (MODE == M_W8A8) {
           *as_global_w(reinterpret_cast<f32x4*>(a.og + (size_t)m * 2048 + h * 256 + d0)) = o;
         } else {   // elements 4 (j % 4) + td of chunk 16 h + 4 wave + j / 4
-          const int c = 16 * h + 4 * wave + (j >> 2);
-          float* p = a.og + (((size_t)(m >> 4) * pf_frags(2048) + pf_visit(2048, c)) * 64 + (m & 15)) * 4 + (j & 3);
 #pragma unroll
-          for (int td = 0; td < 4; ++td) as_global_w(p)[64 * td] = o[td];
+          for (int td = 0; td < 4; ++td)
+            as_global_w(a.og)[pf_frag_f32(2048, m, 16 * h + 4 * wave + (j >> 2), 4 * (j & 3) + td)] = o[td];
         }
       }
     }
@@ -871,27 +1035,44 @@ hipError_t pf_norm(const PfNorm& a, int mode, hipStream_t s) {
 }
 
 namespace {
-template <int MODE, int K, int TA, int EPI>
-hipError_t gemm_launch(const PfGemm& a, hipStream_t s) {
-  const int ntile = (a.M + 15) / 16;
-  const dim3 grid(a.rows / (16 * TA), (ntile + 3) / 4);
-  pf_gemm_kernel<MODE, K, TA, 1, EPI><<<grid, 256, 0, s>>>(a);
+// Token tiles per workgroup: as few as keep the grid within one round of two workgroups per CU
+// (a second, nearly empty round would cost as much as the first), at least `least`.
+int tiles_per_wg(int row_tiles, int ntile, int least) {
+  const int ny = 512 / row_tiles > 0 ? 512 / row_tiles : 1;
+  int t = (ntile + ny - 1) / ny;
+  t = (t + least - 1) / least * least;
+  return t;
+}
+template <int K, int TA, int EPI>
+hipError_t gemm_i8(const PfGemm& a, hipStream_t s) {
+  const int ntile = (a.M + 15) / 16, rt = a.rows / (16 * TA), tpw = tiles_per_wg(rt, ntile, 4);
+  pf_gemm_i8_kernel<K, TA, EPI><<<dim3(rt, (ntile + tpw - 1) / tpw), 256, 0, s>>>(a, tpw);
   return hipGetLastError();
 }
-template <int MODE>
-hipError_t gemm_mode(const PfGemm& a, int K, PfEpi epi, hipStream_t s) {
-  if (K == 1024 && epi == PF_INPROJ) return gemm_launch<MODE, 1024, 4, PF_INPROJ>(a, s);
-  if (K == 1024 && epi == PF_STORE) return gemm_launch<MODE, 1024, 4, PF_STORE>(a, s);
-  if (K == 1024 && epi == PF_SWIGLU) return gemm_launch<MODE, 1024, 4, PF_SWIGLU>(a, s);
-  if (K == 2048 && epi == PF_RESID) return gemm_launch<MODE, 2048, 2, PF_RESID>(a, s);
-  if (K == 3584 && epi == PF_RESID) return gemm_launch<MODE, 3584, 2, PF_RESID>(a, s);
-  return hipErrorInvalidValue;
+template <int K, int RT, int KS, int EPI>
+hipError_t gemm_f32(const PfGemm& a, hipStream_t s) {
+  const int ntile = (a.M + 31) / 32, rt = a.rows / (32 * RT), tpw = tiles_per_wg(rt, ntile, 1);
+  pf_gemm_f32_kernel<K, RT, KS, EPI><<<dim3(rt, (ntile + tpw - 1) / tpw), 64 * RT * KS, 0, s>>>(a, tpw);
+  return hipGetLastError();
 }
 }  // namespace
 
 hipError_t pf_gemm(const PfGemm& a, int K, PfEpi epi, int mode, hipStream_t s) {
   if (a.M < 1 || a.M > kPfGroup || a.rows % 64 != 0 || a.nseg < 1 || a.nseg > 3) return hipErrorInvalidValue;
-  return mode == M_W8A8 ? gemm_mode<M_W8A8>(a, K, epi, s) : gemm_mode<M_W8A16>(a, K, epi, s);
+  if (mode == M_W8A8) {
+    if (K == 1024 && epi == PF_INPROJ) return gemm_i8<1024, 4, PF_INPROJ>(a, s);
+    if (K == 1024 && epi == PF_STORE) return gemm_i8<1024, 4, PF_STORE>(a, s);
+    if (K == 1024 && epi == PF_SWIGLU) return gemm_i8<1024, 4, PF_SWIGLU>(a, s);
+    if (K == 2048 && epi == PF_RESID) return gemm_i8<2048, 1, PF_RESID>(a, s);
+    if (K == 3584 && epi == PF_RESID) return gemm_i8<3584, 1, PF_RESID>(a, s);
+  } else {
+    if (K == 1024 && epi == PF_INPROJ) return gemm_f32<1024, 2, 2, PF_INPROJ>(a, s);
+    if (K == 1024 && epi == PF_STORE) return gemm_f32<1024, 2, 2, PF_STORE>(a, s);
+    if (K == 1024 && epi == PF_SWIGLU) return gemm_f32<1024, 2, 2, PF_SWIGLU>(a, s);
+    if (K == 2048 && epi == PF_RESID) return gemm_f32<2048, 1, 4, PF_RESID>(a, s);
+    if (K == 3584 && epi == PF_RESID) return gemm_f32<3584, 1, 8, PF_RESID>(a, s);
+  }
+  return hipErrorInvalidValue;
 }
 
 hipError_t pf_conv(const PfConv& a, hipStream_t s) {
@@ -899,7 +1080,7 @@ hipError_t pf_conv(const PfConv& a, hipStream_t s) {
   return hipGetLastError();
 }
 hipError_t pf_scan(const PfScan& a, hipStream_t s) {
-  pf_scan_kernel<<<256, 64, 0, s>>>(a);
+  pf_scan_kernel<<<256, 256, 0, s>>>(a);
   return hipGetLastError();
 }
 hipError_t pf_gated(const PfGated& a, int mode, hipStream_t s) {

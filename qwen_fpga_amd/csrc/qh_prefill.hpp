@@ -10,23 +10,29 @@
 namespace qh {
 
 constexpr int kPfTile = 16;       // tokens per MFMA tile
-constexpr int kPfGroup = 512;     // tokens per group: the largest M of every launch
+constexpr int kPfGroup = 1024;    // the largest group (M of every launch)
+constexpr int kPfSlots = 2;       // groups in flight
 constexpr int kPfMaxPos = kAttnShortMax;   // positions the grouped attention covers (16-position splits)
 
-// Activations in MFMA fragment order.  For token tile tt = m / 16, j = m % 16:
-//   W8A8   int8: 16-element chunk c of token j at byte (((tt * K/64 + c/4) * 4 + c%4) * 16 + j) * 16
-//   W8A16  fp32: element 16 c + 4 i + g of token j at float
-//          ((tt * pf_frags(K) + pf_visit(c)) * 64 + 16 g + j) * 4 + i
-// so that the operand of one MFMA step is 1 KiB of consecutive memory, 16 bytes per lane.
-// The fp32 chunks stand in the order the C16 sum visits them: chunk c belongs to lane l = c % 64
-// of the 64-lane tree, lanes are visited in bit-reversed order (so that the tree needs a stack of
-// six partial sums instead of 64), and a lane's chunks l, l + 64, ... follow one another.
+// Activations in MFMA fragment order: the operand of one MFMA step is consecutive memory, 16 bytes
+// per lane.
+//   W8A8   int8: 16-element chunk c of token m (tile tt = m / 16, j = m % 16) at byte
+//          (((tt * K/64 + c/4) * 4 + c%4) * 16 + j) * 16
+//   W8A16  fp32: pf_frag_f32, token tiles of 32.  The chunks stand in the order the C16 sum visits
+//          them: chunk c belongs to lane l = c % 64 of the 64-lane tree, lanes are visited in
+//          bit-reversed order (so that the tree needs a stack of six partial sums instead of 64),
+//          and a lane's chunks l, l + 64, ... follow one another.
 __host__ __device__ constexpr int pf_bitrev6(int l) {
   return ((l & 1) << 5) | ((l & 2) << 3) | ((l & 4) << 1) | ((l & 8) >> 1) | ((l & 16) >> 3) | ((l & 32) >> 5);
 }
 __host__ __device__ constexpr int pf_nch(int K) { return (K + 1023) / 1024; }
 __host__ __device__ constexpr int pf_frags(int K) { return 64 * pf_nch(K); }
 __host__ __device__ constexpr int pf_visit(int K, int c) { return pf_bitrev6(c & 63) * pf_nch(K) + (c >> 6); }
+// float index of element e of chunk c of token m: lane 32 (e % 2) + m % 32, element (e / 2) % 4 of
+// its 16 bytes, half e / 8 of the chunk's two steps
+__host__ __device__ constexpr size_t pf_frag_f32(int K, int m, int c, int e) {
+  return ((((size_t)(m >> 5) * pf_frags(K) + pf_visit(K, c)) * 2 + (e >> 3)) * 64 + 32 * (e & 1) + (m & 31)) * 4 + ((e >> 1) & 3);
+}
 
 enum PfEpi : int {
   PF_INPROJ = 0,   // qkv rows stored, z rows through SiLU

@@ -1,7 +1,7 @@
 """Prompts run in groups (qh_prefill.hip) leave what feeding them token by token leaves, bit for
 bit: the recurrent, conv and KV state, the next token and its logits.  Lengths at the edges of the
-MFMA tile (16 tokens), of the group (512), of the positions the grouped attention covers (2048),
-and prompts that start inside a tile.  The prompt's last token always runs on the executor, so n
+MFMA tiles (16 and 32 tokens) and of the scan's blocks (8), of one group (512, then two halves), of
+the positions the grouped attention covers (2048), and prompts that start inside a tile.  The prompt's last token always runs on the executor, so n
 tokens take the grouped path for n - 1 of them."""
 import numpy as np
 import pytest
@@ -44,7 +44,7 @@ def test_prompt_in_groups_equals_token_by_token(q, blob, torch_cuda, mode, exec_
         e.set_exec(q.EXEC_GRAPH if exec_kind == "graph" else q.EXEC_PERSISTENT)
         r = rng(77 + mode)
         ids = lambda n: r.integers(0, q.VOCAB, size=n).astype(np.int32).tolist()
-        lens = [[14], [16], [17], [18], [66], [3, 20], [21, 40, 2, 15]]
+        lens = [[9], [14], [16], [17], [18], [33], [34], [66], [3, 20], [21, 40, 2, 15]]
         if exec_kind == "persistent":
             lens += [[129], [513], [514], [30, 530]]
         for ls in lens:
