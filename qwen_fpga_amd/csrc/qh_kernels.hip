@@ -65,6 +65,30 @@ hipError_t launch_gemv(const GemvArgs& a, int waves_per_block, hipStream_t s) {
   }
 }
 
+// The attention layer op's q, k, v projections; the last workgroup also stores the RoPE row and the
+// slot that the attention launch reads (two launches of their own cost 2.6 us and their gaps).
+template <int MODE>
+__global__ __launch_bounds__(256) void attn_qkv_kernel(const GemvArgs a, const AttnSetup u) {
+  if (blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x < 64) u.rope_out[threadIdx.x] = u.rope.v[threadIdx.x];
+    if (threadIdx.x == 64) {
+      u.ints_out[0] = u.T;
+      u.ints_out[1] = 0;
+    }
+  }
+  PlainIO io{a.done};
+  gemv_body<1, MODE, P_LOAD, 8>(a, blockIdx.x, gridDim.x, io, a.tokv);
+}
+hipError_t launch_attn_qkv(const GemvArgs& a, const AttnSetup& u, hipStream_t s) {
+  if (a.K != QH_HIDDEN || a.prologue != P_LOAD || a.rows_per_batch != 8) return hipErrorInvalidValue;
+  const int grid = (a.seg[a.nseg - 1].batch0 + a.seg[a.nseg - 1].nbatch + 3) / 4;
+  if (a.mode == M_W8A8)
+    attn_qkv_kernel<M_W8A8><<<grid, 256, 0, s>>>(a, u);
+  else
+    attn_qkv_kernel<M_W8A16><<<grid, 256, 0, s>>>(a, u);
+  return hipGetLastError();
+}
+
 __global__ __launch_bounds__(256) void head_kernel(const HeadArgs a) {
   PlainIO io{a.done};
   head_body<true>(a, blockIdx.x, gridDim.x, io, a.logits);
@@ -187,13 +211,9 @@ hipError_t launch_embed(float* h, const int8_t* w, const float* sc, int tok, int
 }
 
 // one wave: C16 sum of squares over n, then the (1+w) or gated scaling.
-// One vector of n per workgroup: workgroup b normalises x[b n .. b n + n) (w shared).
 __global__ void rmsnorm_kernel(float* y, const float* x, const float* w, const float* z, int n, float eps,
                                int gated) {
   const int lane = threadIdx.x;
-  y += (size_t)blockIdx.x * n;
-  x += (size_t)blockIdx.x * n;
-  if (z != nullptr) z += (size_t)blockIdx.x * n;
   const int nchunk = (n + 15) / 16;
   float ss = 0.0f;
   for (int c = lane; c < nchunk; c += 64)
@@ -204,8 +224,8 @@ __global__ void rmsnorm_kernel(float* y, const float* x, const float* w, const f
     y[i] = gated ? ((x[i] * inv) * w[i]) * dev_silu(z[i]) : (x[i] * inv) * (1.0f + w[i]);
 }
 hipError_t launch_rmsnorm(float* y, const float* x, const float* w, const float* z, int n, float eps,
-                          int gated, hipStream_t s, int groups) {
-  rmsnorm_kernel<<<groups, 64, 0, s>>>(y, x, w, z, n, eps, gated);
+                          int gated, hipStream_t s) {
+  rmsnorm_kernel<<<1, 64, 0, s>>>(y, x, w, z, n, eps, gated);
   return hipGetLastError();
 }
 
@@ -245,24 +265,99 @@ __global__ void conv1d_kernel(float* out, const float* in, float* state, const f
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < C) conv1d_channel(out, in, state, w, c);
 }
-// The DeltaNet step's inputs of the delta rule (deltanet.hpp:155-165): the short conv + SiLU of
-// the 6144 qkv channels, and per head beta = sigmoid(b), g = -exp(A_log) softplus(a + dt_bias)
-// into gb = g[16] | beta[16] (threads 6144 .. 6159).
-__global__ void dn_step_pre_kernel(float* convd, float* gb, const float* qkv, float* state, const float* cw,
-                                   const float* b, const float* a, const float* A_log, const float* dt_bias) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < QH_CONV_DIM) {
-    conv1d_channel(convd, qkv, state, cw, c);
-  } else if (c < QH_CONV_DIM + QH_LH) {
-    const int h = c - QH_CONV_DIM;
-    gb[QH_LH + h] = dev_sigmoid(b[h]);
-    gb[h] = -dev_expf(A_log[h]) * dev_softplus(a[h] + dt_bias[h]);
+// The DeltaNet recurrent step between the projections (deltanet.hpp:154-179), one head per
+// workgroup: the short conv + SiLU of the head's 384 channels and its gates beta = sigmoid(b),
+// g = -exp(A_log) softplus(a + dt_bias) into LDS, the delta rule over the head's 128 x 128 state
+// (deltanet_body's layout and operations: 256 threads per 32 columns), the gated RMSNorm.  Latency
+// bound: the state's 64 KiB per workgroup are in flight while the conv runs.  As three launches
+// (conv, delta rule, norm) the kernels took 10.8 us and a call 20.6.
+__global__ __launch_bounds__(1024) void dn_step_kernel(const DnStepArgs a) {
+  __shared__ __attribute__((aligned(16))) float qkv[3 * 128];   // the head's q, k, v
+  __shared__ float gb[2];
+  __shared__ __attribute__((aligned(16))) float ol[128];
+  const int t = threadIdx.x, lane = t & 63, h = blockIdx.x;
+  const int kg = lane & 7, v = (t >> 6) * 8 + (lane >> 3);
+  float* Sh = a.S + (size_t)h * 128 * 128;
+  float s[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) s[i] = as_global(Sh)[(kg * 16 + i) * 128 + v];
+  if (t < 384) {   // channel t of the head: q, k or v (each 2048 channels of the layer)
+    const int c = (t >> 7) * 2048 + h * 128 + (t & 127);
+    f32x4* stp = reinterpret_cast<f32x4*>(a.conv_state + (size_t)c * 4);
+    float w0, w1, w2, w3 = as_global(a.qkv)[c], tap[4];
+    if ((reinterpret_cast<uintptr_t>(a.conv_state) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.conv_w) & 15) == 0) {
+      const f32x4 st = *as_global(stp), w = *as_global(reinterpret_cast<const f32x4*>(a.conv_w + (size_t)c * 4));
+      w0 = st[1], w1 = st[2], w2 = st[3];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) tap[k] = w[k];
+      *as_global_w(stp) = f32x4{w0, w1, w2, w3};
+    } else {   // pointers with no more than a float's alignment
+      float* st = a.conv_state + (size_t)c * 4;
+      w0 = st[1], w1 = st[2], w2 = st[3];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) tap[k] = a.conv_w[(size_t)c * 4 + k];
+      st[0] = w0, st[1] = w1, st[2] = w2, st[3] = w3;
+    }
+    float acc = 0.0f;
+    acc = acc + w0 * tap[0];
+    acc = acc + w1 * tap[1];
+    acc = acc + w2 * tap[2];
+    acc = acc + w3 * tap[3];
+    as_lds_w(qkv)[t] = dev_silu(acc);
+  } else if (t == 384) {
+    as_lds_w(gb)[0] = -dev_expf(as_global(a.A_log)[h]) * dev_softplus(as_global(a.a)[h] + as_global(a.dt_bias)[h]);
+  } else if (t == 448) {
+    as_lds_w(gb)[1] = dev_sigmoid(as_global(a.b)[h]);
   }
+  lds_barrier();
+  float qk[2][16];
+  load16l(qkv + 16 * kg, qk[0]);
+  load16l(qkv + 128 + 16 * kg, qk[1]);
+  const float vt = as_lds(qkv)[256 + v];
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {   // l2norm (deltanet.hpp:134); q also scaled by 1 / sqrt(128)
+    float ss = dot16_f32(qk[w], qk[w], 0.0f);
+    ss = xor_sum<8>(ss);
+    const float inv = 1.0f / sqrtf(ss + 1e-6f);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) qk[w][e] = qk[w][e] * inv;
+  }
+  const float sc = 1.0f / sqrtf(128.0f);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) qk[0][e] = qk[0][e] * sc;
+  const float gexp = dev_expf(as_lds(gb)[0]), beta = as_lds(gb)[1];
+  float p = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {   // sweep A
+    s[i] = s[i] * gexp;
+    p = p + s[i] * qk[1][i];
+  }
+  p = xor_sum<8>(p);
+  const float d = (vt - p) * beta;
+  p = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {   // sweep B: reads the updated S
+    s[i] = s[i] + qk[1][i] * d;
+    p = p + s[i] * qk[0][i];
+    as_global_w(Sh)[(kg * 16 + i) * 128 + v] = s[i];
+  }
+  p = xor_sum<8>(p);
+  if (kg == 0) as_lds_w(ol)[v] = p;
+  lds_barrier();
+  if (t >= 128) return;
+  // per-head gated RMSNorm with silu(z) (deltanet.hpp:177-179), rmsnorm_kernel's order
+  float ss = 0.0f;
+  if (lane < 8) {
+    float x[16];
+    load16l(ol + 16 * lane, x);
+    ss = dot16_f32(x, x, 0.0f);
+  }
+  ss = xor_sum<64>(ss);
+  const float inv = 1.0f / sqrtf(ss / 128.0f + 1e-6f);
+  a.out[h * 128 + t] = ((as_lds(ol)[t] * inv) * as_global(a.nw)[t]) * dev_silu(as_global(a.z)[h * 128 + t]);
 }
-hipError_t launch_dn_step_pre(float* convd, float* gb, const float* qkv, float* state, const float* cw,
-                              const float* b, const float* a, const float* A_log, const float* dt_bias,
-                              hipStream_t s) {
-  dn_step_pre_kernel<<<(QH_CONV_DIM + QH_LH + 255) / 256, 256, 0, s>>>(convd, gb, qkv, state, cw, b, a, A_log, dt_bias);
+hipError_t launch_dn_step(const DnStepArgs& a, hipStream_t s) {
+  dn_step_kernel<<<QH_LH, 1024, 0, s>>>(a);
   return hipGetLastError();
 }
 hipError_t launch_conv1d(float* out, const float* in, float* state, const float* w, int C, hipStream_t s) {
@@ -282,21 +377,39 @@ hipError_t launch_apply_rope(float* x, const float* cs, const float* sn, hipStre
   return hipGetLastError();
 }
 
-__global__ void quant_kernel(int8_t* q, float* sx, const float* x, int n) {
-  __shared__ float sm[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  float am = 0.0f;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) am = fmaxf(am, fabsf(x[i]));
+// One workgroup (the vectors are a few thousand elements).  Up to kQuantRegs * 1024 elements stay in
+// registers between the maximum and the quotients; longer vectors are read twice.  (256 threads and
+// two passes took 5.7 us at 3584 elements, this 3.4.)
+constexpr int kQuantRegs = 4;
+__global__ __launch_bounds__(1024) void quant_kernel(int8_t* q, float* sx, const float* x, int n) {
+  __shared__ float sm[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  float v[kQuantRegs], am = 0.0f;
+#pragma unroll
+  for (int k = 0; k < kQuantRegs; ++k) {
+    const int i = t + 1024 * k;
+    v[k] = i < n ? as_global(x)[i] : 0.0f;
+  }
+#pragma unroll
+  for (int k = 0; k < kQuantRegs; ++k) am = fmaxf(am, fabsf(v[k]));
+  for (int i = t + 1024 * kQuantRegs; i < n; i += 1024) am = fmaxf(am, fabsf(x[i]));
   am = xor_max<64>(am);
-  if (lane == 0) sm[wave] = am;
-  __syncthreads();
-  am = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
+  if (lane == 0) as_lds_w(sm)[wave] = am;
+  lds_barrier();
+  am = 0.0f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) am = fmaxf(am, as_lds(sm)[w]);
   const float s = quant_scale(am);
-  for (int i = threadIdx.x; i < n; i += blockDim.x) q[i] = (int8_t)quant_one(x[i], s);
-  if (threadIdx.x == 0) *sx = s;
+#pragma unroll
+  for (int k = 0; k < kQuantRegs; ++k) {
+    const int i = t + 1024 * k;
+    if (i < n) as_global_w(q)[i] = (int8_t)quant_one(v[k], s);
+  }
+  for (int i = t + 1024 * kQuantRegs; i < n; i += 1024) q[i] = (int8_t)quant_one(x[i], s);
+  if (t == 0) *sx = s;
 }
 hipError_t launch_quant(int8_t* q, float* sx, const float* x, int n, hipStream_t s) {
-  quant_kernel<<<1, 256, 0, s>>>(q, sx, x, n);
+  quant_kernel<<<1, 1024, 0, s>>>(q, sx, x, n);
   return hipGetLastError();
 }
 
@@ -326,7 +439,7 @@ __device__ __forceinline__ void qr_load4(const uint16_t* p, float (&v)[4]) {
   v[2] = __uint_as_float(t[1] << 16);
   v[3] = __uint_as_float(t[1] & 0xffff0000u);
 }
-template <typename T>
+template <typename T, int REGS>
 __global__ __launch_bounds__(256) void quant_rows_kernel(int8_t* q, float* scale, const T* w, int rows, int cols,
                                                          int vec) {
   const int lane = threadIdx.x & 63;
@@ -336,10 +449,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(int8_t* q, float* scale
   int8_t* qr = q + (size_t)row * cols;
   float am = 0.0f;
   bool bad = false;
-  if (vec) {   // cols % 4 == 0, cols <= kQRowRegs * 256, aligned
-    float v[kQRowRegs][4];
+  if (vec) {   // cols % 4 == 0, cols <= REGS * 256, aligned
+    float v[REGS][4];
 #pragma unroll
-    for (int c = 0; c < kQRowRegs; ++c) {
+    for (int c = 0; c < REGS; ++c) {
       const int i = 4 * (lane + 64 * c);
       if (i < cols) {
         qr_load4(wr + i, v[c]);
@@ -356,7 +469,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(int8_t* q, float* scale
     const float s = bad ? __builtin_nanf("") : quant_scale(am);
     const float rs = 1.0f / s;
 #pragma unroll
-    for (int c = 0; c < kQRowRegs; ++c) {
+    for (int c = 0; c < REGS; ++c) {
       const int i = 4 * (lane + 64 * c);
       if (i < cols) {
         int t[4];
@@ -386,7 +499,11 @@ hipError_t launch_quant_rows_t(int8_t* q, float* scale, const T* w, int rows, in
   const size_t in_align = sizeof(T) == 4 ? 16 : 8;
   const int vec = cols % 4 == 0 && cols <= kQRowRegs * 256 && reinterpret_cast<uintptr_t>(w) % in_align == 0 &&
                   reinterpret_cast<uintptr_t>(q) % 4 == 0;
-  quant_rows_kernel<T><<<(rows + 3) / 4, 256, 0, s>>>(q, scale, w, rows, cols, vec);
+  const int grid = (rows + 3) / 4;
+  if (cols <= 1024)
+    quant_rows_kernel<T, 4><<<grid, 256, 0, s>>>(q, scale, w, rows, cols, vec);
+  else
+    quant_rows_kernel<T, kQRowRegs><<<grid, 256, 0, s>>>(q, scale, w, rows, cols, vec);
   return hipGetLastError();
 }
 hipError_t launch_quant_rows(int8_t* q, float* scale, const float* w, int rows, int cols, hipStream_t s) {
@@ -411,15 +528,6 @@ hipError_t launch_fixed_dequant(int32_t* yq, const int32_t* acc, const int32_t* 
                                 hipStream_t s) {
   if (n <= 0 || shift < 1 || shift > 62 || outw < 1 || outw > 32) return hipErrorInvalidValue;
   fixed_dequant_kernel<<<(n + 255) / 256, 256, 0, s>>>(yq, acc, mult, n, shift, outw);
-  return hipGetLastError();
-}
-
-__global__ void set_ints_kernel(int* dst, int a, int b) {
-  dst[0] = a;
-  dst[1] = b;
-}
-hipError_t launch_set_ints(int* dst, int a, int b, hipStream_t s) {
-  set_ints_kernel<<<1, 1, 0, s>>>(dst, a, b);
   return hipGetLastError();
 }
 

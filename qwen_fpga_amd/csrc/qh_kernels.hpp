@@ -199,6 +199,29 @@ struct DnArgs {
 
 struct Floats64 { float v[64]; };
 
+// What the attention layer op's q, k, v launch stores beside its rows (launch_attn_qkv).
+struct AttnSetup {
+  Floats64 rope;               // cos[32] | sin[32] of this position
+  float* rope_out = nullptr;
+  int* ints_out = nullptr;     // T, then 0 (the RoPE row index)
+  int T = 0;
+};
+
+// The DeltaNet recurrent step between the projections in one launch (launch_dn_step).
+struct DnStepArgs {
+  float* out = nullptr;            // [2048]
+  const float* qkv = nullptr;      // [6144]
+  const float* z = nullptr;        // [2048]
+  const float* b = nullptr;        // [16]
+  const float* a = nullptr;        // [16]
+  const float* conv_w = nullptr;   // [6144][4]
+  const float* A_log = nullptr;
+  const float* dt_bias = nullptr;
+  const float* nw = nullptr;       // [128]
+  float* S = nullptr;              // [16][128][128]
+  float* conv_state = nullptr;     // [6144][4]
+};
+
 // One stage of a decode step: the arguments a per-stage kernel would get, and
 // which body runs them.  The three K > 1024 GEMVs use one row per wave batch
 // (1024 rows = 1024 batches), so every wave of a 256-workgroup grid streams.
@@ -284,12 +307,10 @@ hipError_t launch_advance(StepCtl* ctl, const int* prompt, int* out_ids, hipStre
 // small op kernels
 hipError_t launch_embed(float* h, const int8_t* w, const float* sc, int tok, int in, hipStream_t s);
 hipError_t launch_rmsnorm(float* y, const float* x, const float* w, const float* z, int n, float eps,
-                          int gated, hipStream_t s,
-                          int groups = 1);
+                          int gated, hipStream_t s);
 hipError_t launch_l2norm(float* v, int n, hipStream_t s);
-hipError_t launch_dn_step_pre(float* convd, float* gb, const float* qkv, float* state, const float* cw,
-                              const float* b, const float* a, const float* A_log, const float* dt_bias,
-                              hipStream_t s);
+hipError_t launch_dn_step(const DnStepArgs& a, hipStream_t s);
+hipError_t launch_attn_qkv(const GemvArgs& a, const AttnSetup& u, hipStream_t s);
 hipError_t launch_conv1d(float* out, const float* in, float* state, const float* w, int C,
                          hipStream_t s);
 hipError_t launch_apply_rope(float* x, const float* cs, const float* sn, hipStream_t s);
@@ -298,7 +319,6 @@ hipError_t launch_fixed_dequant(int32_t* yq, const int32_t* acc, const int32_t* 
                                 hipStream_t s);
 hipError_t launch_quant_rows(int8_t* q, float* scale, const float* w, int rows, int cols, hipStream_t s);
 hipError_t launch_quant_rows_bf16(int8_t* q, float* scale, const uint16_t* w, int rows, int cols, hipStream_t s);
-hipError_t launch_set_ints(int* dst, int a, int b, hipStream_t s);
 hipError_t launch_set_int(int* dst, int v, hipStream_t s);
 hipError_t launch_dn_gather(float* convd, float* gb, const float* q, const float* k, const float* v, const float* g,
                             const float* beta, float gs, float bs, int nq, int nv, int nh, hipStream_t s);

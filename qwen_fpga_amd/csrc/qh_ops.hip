@@ -134,6 +134,18 @@ Seg seg_i8(const int8_t* w, const float* sw, int rows, int batch0, float* out, i
   return g;
 }
 
+// Rows a wave reduces together.  Eight rows share the activation's staging and reduction, but the
+// grid is rows / R waves: below one wave per SIMD (1024) the chip is idle and each wave's loads queue
+// behind one another.  Measured (us per call, R = 8 / 4 / 1): 1024x3584 W8A8 7.8 / 6.7 / 6.2, W8A16
+// 9.3 / 7.5 / 6.6; 4096x3584 W8A8 8.2 / 7.7 / 9.6; 6144x3584 W8A8 8.9 / 10.9 / 11.2; 32768x3584 W8A16
+// 35.2 / 27.4 / 52.8 (eight rows of four fp32-multiplied chunks do not fit the registers of two waves
+// per SIMD); 32768x1024 W8A16 12.8 / 15.9 / 41.1.
+int gemv_rows(int rows, int K, int mode) {
+  if (rows <= 2048) return 1;
+  if (K > 2048) return mode == M_W8A16 || rows <= 4096 ? 4 : 8;
+  return rows <= 8192 ? 4 : 8;
+}
+
 int check_gemv_shape(int out, int in) {
   if (out <= 0 || in <= 0 || in % 16 != 0 || in > 4096) return QH_EINVAL;
   return QH_OK;
@@ -188,9 +200,9 @@ int deltanet_layer(float* out, const float* x, const qh_tensor* qkv_w, const qh_
   c.nw = gate_norm_w;
   c.z = zb;
   c.nseg = 1;
-  c.rows_per_batch = 4;
-  c.seg[0] = seg_i8(out_w->w_i8, out_w->scale, kHidden, 0, out, E_STORE, 4);
-  QH_HIP(launch_gemv(c, 1, s));
+  c.rows_per_batch = 1;   // 1024 rows: a row per wave fills the chip (gemv_rows)
+  c.seg[0] = seg_i8(out_w->w_i8, out_w->scale, kHidden, 0, out, E_STORE, 1);
+  QH_HIP(launch_gemv(c, 4, s));
   return QH_OK;
 }
 
@@ -229,11 +241,12 @@ int attention_layer(float* out, const float* x, const qh_tensor* q_w, const qh_t
   a.seg[0] = seg_i8(q_w->w_i8, q_w->scale, kQProj, 0, qg, E_STORE);
   a.seg[1] = seg_i8(k_w->w_i8, k_w->scale, kKVProj, a.seg[0].nbatch, kraw, E_STORE);
   a.seg[2] = seg_i8(v_w->w_i8, v_w->scale, kKVProj, a.seg[0].nbatch + a.seg[1].nbatch, vraw, E_STORE);
-  QH_HIP(launch_gemv(a, 4, s));
-  Floats64 r;
-  rope_row(pos, r.v);
-  QH_HIP(launch_set_floats(rope, r, 64, s));
-  QH_HIP(launch_set_ints(ints, T, 0, s));
+  AttnSetup u;   // the launch also stores the RoPE row, the slot and the row index for the attention
+  rope_row(pos, u.rope.v);
+  u.rope_out = rope;
+  u.ints_out = ints;
+  u.T = T;
+  QH_HIP(launch_attn_qkv(a, u, s));
   AttnArgs at;
   at.qkv = qkv;
   at.qn = q_norm;
@@ -257,9 +270,9 @@ int attention_layer(float* out, const float* x, const qh_tensor* q_w, const qh_t
   c.prologue = P_LOAD;
   c.x = og;
   c.nseg = 1;
-  c.rows_per_batch = 4;
-  c.seg[0] = seg_i8(o_w->w_i8, o_w->scale, kHidden, 0, out, E_STORE, 4);
-  QH_HIP(launch_gemv(c, 1, s));
+  c.rows_per_batch = 1;   // 1024 rows: a row per wave fills the chip (gemv_rows)
+  c.seg[0] = seg_i8(o_w->w_i8, o_w->scale, kHidden, 0, out, E_STORE, 1);
+  QH_HIP(launch_gemv(c, 4, s));
   return QH_OK;
 }
 
@@ -296,9 +309,9 @@ int mlp_layer(float* out, const float* x, const qh_tensor* gate_w, const qh_tens
   c.prologue = P_LOAD;
   c.x = act;
   c.nseg = 1;
-  c.rows_per_batch = 4;
-  c.seg[0] = seg_i8(down_w->w_i8, down_w->scale, kHidden, 0, out, E_STORE, 4);
-  QH_HIP(launch_gemv(c, 1, s));
+  c.rows_per_batch = 1;   // 1024 rows: a row per wave fills the chip (gemv_rows)
+  c.seg[0] = seg_i8(down_w->w_i8, down_w->scale, kHidden, 0, out, E_STORE, 1);
+  QH_HIP(launch_gemv(c, 4, s));
   return QH_OK;
 }
 
@@ -329,7 +342,8 @@ int qh_gemv_i8(float* y, const int8_t* w, const float* scale, const float* x, in
   a.prologue = P_LOAD;
   a.x = x;
   a.nseg = 1;
-  a.seg[0] = seg_i8(w, scale, out, 0, y, E_STORE);
+  a.rows_per_batch = gemv_rows(out, in, a.mode);
+  a.seg[0] = seg_i8(w, scale, out, 0, y, E_STORE, a.rows_per_batch);
   return hip_status(launch_gemv(a, 4, S(stream)));
 }
 
@@ -453,7 +467,8 @@ int qh_delta_rule_layer(const float* q, const float* k, const float* v, const fl
   return hip_status(launch_deltanet(d, s));
 }
 
-// The scratch of qh_deltanet_step: post-conv qkv, g | beta, the delta-rule output.
+// The workspace qh_deltanet_step requires: room for post-conv qkv, g | beta and the delta-rule output
+// (the step keeps them in LDS now; the size callers ask for and pass stays).
 constexpr size_t kDnStepWorkspace = rnd(4 * kConvDim) + rnd(4 * 2 * kLH) + rnd(4 * kLH * kLV);
 size_t qh_deltanet_step_workspace(void) { return kDnStepWorkspace; }
 
@@ -464,21 +479,19 @@ int qh_deltanet_step(float* out, const float* qkv, const float* z, const float* 
       !workspace)
     return QH_EINVAL;
   if (workspace_bytes < kDnStepWorkspace || (reinterpret_cast<uintptr_t>(workspace) & 255)) return QH_EINVAL;
-  hipStream_t s = S(stream);
-  Scratch sc(s, static_cast<char*>(workspace), workspace_bytes);
-  float* convd = sc.take<float>(kConvDim);
-  float* gb = sc.take<float>(2 * kLH);
-  float* o = sc.take<float>(kLH * kLV);
-  QH_HIP(launch_dn_step_pre(convd, gb, qkv, conv_state, conv_w, b, a, A_log, dt_bias, s));
-  DnArgs d;   // l2norm, q scale, delta rule (deltanet.hpp:166-175)
-  d.convd = convd;
-  d.gb = gb;
+  DnStepArgs d;   // one launch; the workspace the signature carries stays unused
+  d.out = out;
+  d.qkv = qkv;
+  d.z = z;
+  d.b = b;
+  d.a = a;
+  d.conv_w = conv_w;
+  d.A_log = A_log;
+  d.dt_bias = dt_bias;
+  d.nw = gate_norm_w;
   d.S = rec;
-  d.o = o;
-  d.heads = kLH;
-  QH_HIP(launch_deltanet(d, s));
-  // per-head gated RMSNorm with silu(z) (deltanet.hpp:177-179)
-  return hip_status(launch_rmsnorm(out, o, gate_norm_w, z, kLV, kEps, 1, s, kLH));
+  d.conv_state = conv_state;
+  return hip_status(launch_dn_step(d, S(stream)));
 }
 
 int qh_deltanet_layer(float* out, const float* x, const qh_tensor* qkv_w, const qh_tensor* z_w,
@@ -557,7 +570,8 @@ int qh_gemv_i8_w8a8(float* y, int32_t* acc, const int8_t* w, const float* scale,
   a.xq = xq;
   a.sx = sx;
   a.nseg = 1;
-  a.seg[0] = seg_i8(w, scale, out, 0, y, acc ? E_ACC : E_STORE);
+  a.rows_per_batch = gemv_rows(out, in, a.mode);
+  a.seg[0] = seg_i8(w, scale, out, 0, y, acc ? E_ACC : E_STORE, a.rows_per_batch);
   a.seg[0].acc_out = acc;
   return hip_status(launch_gemv(a, 4, S(stream)));
 }
@@ -573,7 +587,8 @@ int qh_matvec_i8(int32_t* y_q, int32_t* acc, const int8_t* w, const int32_t* mul
   a.prologue = P_LOADQ;
   a.xq = xq;
   a.nseg = 1;
-  a.seg[0] = seg_i8(w, nullptr, out, 0, nullptr, E_ACCI);
+  a.rows_per_batch = gemv_rows(out, in, a.mode);
+  a.seg[0] = seg_i8(w, nullptr, out, 0, nullptr, E_ACCI, a.rows_per_batch);
   a.seg[0].acc_out = acc;
   hipStream_t s = S(stream);
   QH_HIP(launch_gemv(a, 4, s));
