@@ -70,7 +70,8 @@ struct qh_engine {
   size_t arena_pairs = 0;
   uint32_t tag_next = 1;         // first unused tag (the arena holds only smaller tags)
   uint32_t tag_start = 1;        // tag_next once the arena is (re)allocated (test hook QH_TAG_START)
-  int* abort_dev = nullptr;      // set by a hand-over wait that gave up
+  int* abort_dev = nullptr;      // set by a hand-over wait that gave up (behind ctl: one copy brings both back)
+  StepCtl* ctl_host = nullptr;   // pinned: where that copy goes, [0] ctl, [1].tok the abort flag
   // Lane-interleaved copies of the fp32 vectors a wave reads 16 elements per
   // lane (norm gains, the DeltaNet gate rows): element e of lane l's chunk of
   // each 1024-element row at (e / 4) * 256 + 4 l + e % 4, so one 16-byte load
@@ -497,9 +498,13 @@ int ensure_prog(qh_engine* e) {
       if (g.kind == SEG_F32 && !(em & kEmF32)) return QH_ESTATE;
     }
   }
+  const size_t n = v.size();
+  for (size_t i = 0; i < n; ++i)   // behind the program: its DeltaNet stages again (PersistArgs::dn_prog)
+    if (v[i].kind == ST_DELTANET) v.push_back(Stage(v[i]));
+  if (v.size() != n + kNLinear) return QH_ESTATE;
   QH_TRY(dalloc(&e->prog[e->mode], v.size()));
   QH_HIP(hipMemcpy(e->prog[e->mode], v.data(), sizeof(Stage) * v.size(), hipMemcpyHostToDevice));
-  e->prog_n = (int)v.size();
+  e->prog_n = (int)n;
   return QH_OK;
 }
 
@@ -510,8 +515,10 @@ constexpr int kUseGraph = 1000;
 
 // One persistent launch: the prompt (already in prompt_dev) through the
 // run_hls loop, n_new greedy tokens at most, token feedback on the device.
-// step0: prompt tokens already processed; tok0 is the next one.
-int run_persist(qh_engine* e, int tok0, int step0, int n_prompt, int n_new, int eos, bool with_logits, StepCtl* out) {
+// step0: prompt tokens already processed; tok0 is the next one.  set_prompt: tok0 is the whole prompt
+// and is not in prompt_dev yet.
+int run_persist(qh_engine* e, int tok0, int step0, int n_prompt, int n_new, int eos, bool with_logits, bool set_prompt,
+                StepCtl* out) {
   QH_TRY(ensure_prog(e));
   hipStream_t s = e->stream;
   // tags of this launch: tag_base + k * kTagsPerToken + stage, k < n_prompt - step0 + n_new
@@ -530,8 +537,7 @@ int run_persist(qh_engine* e, int tok0, int step0, int n_prompt, int n_new, int 
   c.n_new = n_new;
   c.eos = eos;
   c.max_ctx = e->max_ctx;
-  QH_HIP(hipMemcpyAsync(e->ctl, &c, sizeof c, hipMemcpyHostToDevice, s));
-  QH_HIP(hipMemsetAsync(e->abort_dev, 0, sizeof(int), s));
+  QH_HIP(launch_init_persist(e->ctl, c, e->abort_dev, e->prompt_dev, set_prompt ? tok0 : -1, s));
   PersistArgs a;
   // QH_TRACE_FILE=path: completion time of every stage on every workgroup for
   // the first two tokens of this launch, written as text (s_memrealtime ticks).
@@ -556,6 +562,8 @@ int run_persist(qh_engine* e, int tok0, int step0, int n_prompt, int n_new, int 
   a.abort_flag = e->abort_dev;
   a.poll_limit = e->poll_limit;
   a.dn_lds = e->dn_lds ? 1 : 0;
+  a.dn_prog = e->prog[e->mode] + e->prog_n;
+  a.dn_n = kNLinear;
   a.long_ctx = e->max_ctx > kAttnShortMax ? 1 : 0;
   QH_HIP(hipEventRecord(e->launch_ev[0], s));
   if (const hipError_t le = launch_persist(a, e->persist_grid, s); le != hipSuccess) {
@@ -571,10 +579,10 @@ int run_persist(qh_engine* e, int tok0, int step0, int n_prompt, int n_new, int 
   }
   QH_HIP(hipEventRecord(e->launch_ev[1], s));
   e->tag_next += (uint32_t)need;
-  int aborted = 0;
-  QH_HIP(hipMemcpyAsync(out, e->ctl, sizeof *out, hipMemcpyDeviceToHost, s));
-  QH_HIP(hipMemcpyAsync(&aborted, e->abort_dev, sizeof(int), hipMemcpyDeviceToHost, s));
+  QH_HIP(hipMemcpyAsync(e->ctl_host, e->ctl, 2 * sizeof(StepCtl), hipMemcpyDeviceToHost, s));
   QH_HIP(hipStreamSynchronize(s));
+  *out = e->ctl_host[0];
+  const int aborted = e->ctl_host[1].tok;
   if (trace != nullptr) {
     std::vector<uint64_t> hbuf(trace_n);
     const hipError_t ce = hipMemcpy(hbuf.data(), trace, trace_n * sizeof(uint64_t), hipMemcpyDeviceToHost);
@@ -908,7 +916,8 @@ void release(qh_engine* e) {
   void* bufs[] = {e->blob, e->rec, e->conv, e->kc, e->vc, e->h, e->convd, e->zb, e->gb, e->o, e->act,
                   e->og, e->qkv, e->pm, e->pl, e->pacc, e->rope, e->logits, e->part_val,
                   e->part_idx, e->ctl, e->prompt_dev, e->out_dev, e->prog[0], e->prog[1], e->arena,
-                  e->abort_dev, e->lanes};
+                  e->lanes};
+  if (e->ctl_host) (void)hipHostFree(e->ctl_host);
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   for (hipEvent_t ev : e->launch_ev)
@@ -1027,7 +1036,6 @@ int create(const void* blob, size_t blob_len, const char* idx_text, int max_ctx,
   QH_C(dalloc(&e->logits, kVocab));
   QH_C(dalloc(&e->part_val, e->head_grid > 256 ? e->head_grid : 256));
   QH_C(dalloc(&e->part_idx, e->head_grid > 256 ? e->head_grid : 256));
-  QH_C(dalloc(&e->abort_dev, 1));
   if (persist_max_grid(&e->persist_grid) != 0) e->persist_grid = 0;
   // every workgroup holds at most kDnSlots DeltaNet state tiles, one unit per stage
   e->dn_lds = e->persist_grid >= kLH * kDnVQuarters &&
@@ -1035,7 +1043,9 @@ int create(const void* blob, size_t blob_len, const char* idx_text, int max_ctx,
   if (e->persist_grid == 0) e->exec = QH_EXEC_GRAPH;
   QH_C(hip_status(hipEventCreate(&e->launch_ev[0])));
   QH_C(hip_status(hipEventCreate(&e->launch_ev[1])));
-  QH_C(dalloc(&e->ctl, 1));
+  QH_C(dalloc(&e->ctl, 2));
+  e->abort_dev = &e->ctl[1].tok;
+  QH_C(hip_status(hipHostMalloc(reinterpret_cast<void**>(&e->ctl_host), 2 * sizeof(StepCtl))));
   {
     std::vector<float> rope((size_t)max_ctx * 64);
     for (int p = 0; p < max_ctx; ++p) rope_row(p, &rope[(size_t)p * 64]);
@@ -1143,9 +1153,8 @@ int qh_decode_token(qh_engine* e, int tok, float* logits, int* argmax_out) {
   if (tok < 0 || tok >= kVocab) return QH_ERANGE;
   if (e->host_pos >= e->max_ctx) return QH_ERANGE;
   if (e->exec == QH_EXEC_PERSISTENT) {   // one token = a prompt of one, no new tokens
-    QH_HIP(hipMemcpyAsync(e->prompt_dev, &tok, sizeof(int), hipMemcpyHostToDevice, e->stream));
     StepCtl c;
-    const int st = run_persist(e, tok, 0, 1, 0, -1, logits != nullptr, &c);
+    const int st = run_persist(e, tok, 0, 1, 0, -1, logits != nullptr, true, &c);
     if (st != kUseGraph) {
       QH_TRY(st);
       if (logits) QH_HIP(hipMemcpy(logits, e->logits, sizeof(float) * kVocab, hipMemcpyDeviceToHost));
@@ -1183,7 +1192,7 @@ int qh_generate(qh_engine* e, const int* prompt, int n_prompt, int n_new, int eo
   QH_TRY(run_prefill(e, prefill_tokens(e, n_prompt), &step0));
   if (e->exec == QH_EXEC_PERSISTENT) {
     StepCtl c;
-    const int st = run_persist(e, prompt[step0], step0, n_prompt, n_new, eos, false, &c);
+    const int st = run_persist(e, prompt[step0], step0, n_prompt, n_new, eos, false, false, &c);
     if (st != kUseGraph) {
       QH_TRY(st);
       if (c.n_out > 0)

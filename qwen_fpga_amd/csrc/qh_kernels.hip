@@ -546,6 +546,16 @@ hipError_t launch_set_floats(float* dst, const Floats64& v, int n, hipStream_t s
   return hipGetLastError();
 }
 
+__global__ void init_persist_kernel(StepCtl* ctl, const StepCtl c, int* abort_flag, int* prompt, int tok) {
+  *ctl = c;
+  *abort_flag = 0;
+  if (tok >= 0) *prompt = tok;
+}
+hipError_t launch_init_persist(StepCtl* ctl, const StepCtl& c, int* abort_flag, int* prompt, int tok, hipStream_t s) {
+  init_persist_kernel<<<1, 1, 0, s>>>(ctl, c, abort_flag, prompt, tok);
+  return hipGetLastError();
+}
+
 // pos += 1 for a layer-range step (no head / argmax); honours the stop flag.
 __global__ void bump_pos_kernel(StepCtl* c) {
   if (c->done == 0) c->pos = c->pos + 1;

@@ -284,6 +284,8 @@ struct PersistArgs {
   uint64_t* trace = nullptr;    // optional [trace_tokens][nstage][grid][kTraceSlots]: stage marks and end
   int trace_tokens = 0;
   int dn_lds = 0;               // DeltaNet stages keep S in LDS (their unit_base >= 0)
+  const Stage* dn_prog = nullptr;   // with dn_lds: the program's DeltaNet stages alone
+  int dn_n = 0;
   int long_ctx = 0;             // the cache holds more than kAttnShortMax positions: the kernel
                                 // instantiation with the long-context attention (else without it)
 };
@@ -323,6 +325,8 @@ hipError_t launch_set_int(int* dst, int v, hipStream_t s);
 hipError_t launch_dn_gather(float* convd, float* gb, const float* q, const float* k, const float* v, const float* g,
                             const float* beta, float gs, float bs, int nq, int nv, int nh, hipStream_t s);
 hipError_t launch_set_floats(float* dst, const Floats64& v, int n, hipStream_t s);
+// the control block, a cleared abort flag and (tok >= 0) the one prompt token of a persistent launch
+hipError_t launch_init_persist(StepCtl* ctl, const StepCtl& c, int* abort_flag, int* prompt, int tok, hipStream_t s);
 hipError_t launch_bump_pos(StepCtl* ctl, hipStream_t s);
 hipError_t launch_init_gen(StepCtl* ctl, int tok0, int step0, int n_prompt, int n_new, int eos, hipStream_t s);
 

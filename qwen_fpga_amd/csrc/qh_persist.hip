@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kPersistThreads) void persist_kernel(const PersistA
   const int n_prompt = P.ctl->n_prompt, n_new = P.ctl->n_new, eos = P.ctl->eos, max_ctx = P.ctl->max_ctx;
   int argmax = P.ctl->argmax, done = 0, err = 0, aborted = 0;
   const HeadArgs& hd = P.prog[P.nstage - 1].hd;
-  if (P.dn_lds) dn_tiles_copy(P.prog, P.nstage, blk, nblk, true);   // this workgroup's DeltaNet state tiles
+  if (P.dn_lds) dn_tiles_copy(P.dn_prog, P.dn_n, blk, nblk, true);   // this workgroup's DeltaNet state tiles
 
   const uint32_t* progw = reinterpret_cast<const uint32_t*>(P.prog);
   io.desc_next(progw, s_stage[0], kStageWords);   // descriptor of stage 0
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kPersistThreads) void persist_kernel(const PersistA
     }
     if (done) break;
   }
-  if (P.dn_lds) dn_tiles_copy(P.prog, P.nstage, blk, nblk, false);   // the state back to its buffer
+  if (P.dn_lds) dn_tiles_copy(P.dn_prog, P.dn_n, blk, nblk, false);   // the state back to its buffer
   if (blk == 0 && t == 0) {
     StepCtl* c = P.ctl;
     c->tok = tok;

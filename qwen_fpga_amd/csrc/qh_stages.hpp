@@ -1894,9 +1894,13 @@ __device__ __forceinline__ bool deltanet_all(const DnArgs& a, int blk, int nblk,
   return true;
 }
 
-// The LDS tiles of workgroup blk: every DeltaNet stage of the program with a
-// unit on this workgroup copies its slice of S between the state buffer and
-// LDS (to_lds: at the launch start; otherwise back, at its end).
+// The LDS tiles of workgroup blk: every DeltaNet stage of prog with a unit on
+// this workgroup copies its slice of S between the state buffer and LDS
+// (to_lds: at the launch start; otherwise back, at its end).  prog is the list
+// of the DeltaNet stages alone: each step of the walk is a dependent load, and
+// over the whole program's 127 stages the two walks made a one-token launch
+// 40 us longer (same code: an index computed instead of the walk changed the
+// register allocation of the token loop and cost it 2.5%).
 __device__ __forceinline__ void dn_tiles_copy(const Stage* prog, int nstage, int blk, int nblk, bool to_lds) {
   const int t = threadIdx.x, kg = (t & 63) & 7;
   for (int i = 0; i < nstage; ++i) {
