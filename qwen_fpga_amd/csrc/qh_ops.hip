@@ -500,7 +500,7 @@ int qh_delta_rule_layer(const float* q, const float* k, const float* v, const fl
 }
 
 // The workspace qh_deltanet_step requires: room for post-conv qkv, g | beta and the delta-rule output
-// (the step keeps them in LDS now; the size callers ask for and pass stays).
+// (the step keeps them in LDS; an output that overlaps what other heads read is formed here first).
 constexpr size_t kDnStepWorkspace = rnd(4 * kConvDim) + rnd(4 * 2 * kLH) + rnd(4 * kLH * kLV);
 size_t qh_deltanet_step_workspace(void) { return kDnStepWorkspace; }
 
@@ -511,8 +511,21 @@ int qh_deltanet_step(float* out, const float* qkv, const float* z, const float* 
       !workspace)
     return QH_EINVAL;
   if (workspace_bytes < kDnStepWorkspace || (reinterpret_cast<uintptr_t>(workspace) & 255)) return QH_EINVAL;
-  DnStepArgs d;   // one launch; the workspace the signature carries stays unused
-  d.out = out;
+  // One launch, a workgroup per head.  Each reads its inputs and state before it writes its part of
+  // out, but other heads may still be reading theirs: an out that overlaps any of those goes through
+  // the workspace.  (z is read at the element that is written.)
+  const struct {
+    const float* p;
+    size_t n;
+  } in[] = {{qkv, kConvDim}, {b, kLH}, {a, kLH}, {conv_w, kConvDim * kConvK}, {A_log, kLH}, {dt_bias, kLH},
+            {rec, kLH * kLK * kLV}, {conv_state, kConvDim * kConvK}};
+  bool overlap = false;
+  for (const auto& r : in) {
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out), p = reinterpret_cast<uintptr_t>(r.p);
+    overlap |= o < p + sizeof(float) * r.n && p < o + sizeof(float) * kZDim;
+  }
+  DnStepArgs d;
+  d.out = overlap ? static_cast<float*>(workspace) : out;
   d.qkv = qkv;
   d.z = z;
   d.b = b;
@@ -523,7 +536,9 @@ int qh_deltanet_step(float* out, const float* qkv, const float* z, const float* 
   d.nw = gate_norm_w;
   d.S = rec;
   d.conv_state = conv_state;
-  return hip_status(launch_dn_step(d, S(stream)));
+  QH_HIP(launch_dn_step(d, S(stream)));
+  if (overlap) QH_HIP(hipMemcpyAsync(out, workspace, sizeof(float) * kZDim, hipMemcpyDeviceToDevice, S(stream)));
+  return QH_OK;
 }
 
 int qh_deltanet_layer(float* out, const float* x, const qh_tensor* qkv_w, const qh_tensor* z_w,
