@@ -415,86 +415,78 @@ __global__ __launch_bounds__(64 * RT * KS, 2) void pf_gemm_f32_kernel(const PfGe
 
 // ---------------------------------------------------------------------------
 // Short conv + SiLU of the raw qkv rows, then the l2norm of q and k (and q's
-// 1 / sqrt(128)), kConvTok tokens per workgroup.  The convolution is elementwise:
-// thread t takes channel quads t, t + 384, ... so that every load of a wave is
-// consecutive memory, and the results meet in LDS, from which thread c takes
-// channels 16 c .. 16 c + 15 (one k-group of a head) for the norm.  (With 16
-// channels per thread from the start each tap load touched 64 cache lines: 27 us
-// at 512 tokens.)  q and k of (head, token) go to 256 floats in the order the
-// scan reads them: elements 8 e2 + 4 qd .. + 3 of q (e2 = half of a k-group) at
-// 64 qd + 4 e2, k 128 further.
+// 1 / sqrt(128)): kConvTok tokens of kConvCh channels (four heads' q, k or v) per
+// workgroup, so that 63 tokens already make 192 workgroups.  The convolution is
+// elementwise: thread t takes channel quad t, so that every row load of a wave is
+// consecutive memory, and the results meet in LDS, from which thread t takes chunk
+// t % 32 of 16 channels of token t / 32 for the norm.  (With 16 channels per thread
+// from the start each tap load touched 64 cache lines: 27 us at 512 tokens.  With
+// all 6144 channels of two tokens in a workgroup, a launch of 63 tokens was 32
+// workgroups whose tap loads queued behind one another: 12.3 us, where this takes 6.0.)
+// q and k of (head, token) go to 256 floats in the order the scan reads them:
+// elements 8 e2 + 4 qd .. + 3 of q (e2 = half of a k-group) at 64 qd + 4 e2, k 128
+// further.
 // ---------------------------------------------------------------------------
-constexpr int kConvTok = 2;
-__global__ __launch_bounds__(384) void pf_conv_kernel(const PfConv a) {
-  __shared__ __attribute__((aligned(16))) float xl[kConvTok * QH_CONV_DIM];
-  const int t = threadIdx.x, m0 = (int)blockIdx.x * kConvTok;
+constexpr int kConvTok = 4, kConvCh = 512;
+__global__ __launch_bounds__(128) void pf_conv_kernel(const PfConv a) {
+  __shared__ __attribute__((aligned(16))) float xl[kConvTok * kConvCh];
+  const int t = threadIdx.x, m0 = (int)blockIdx.x * kConvTok, ch = (int)blockIdx.y * kConvCh + 4 * t;
+  f32x4 in[3 + kConvTok], tap[4];   // rows m0 - 3 ..; taps of the four channels
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int ch = 4 * (t + 384 * u);
-    f32x4 in[3 + kConvTok], tap[4];   // rows m0 - 3 ..; taps of the four channels
+  for (int e = 0; e < 4; ++e) tap[e] = *as_global(reinterpret_cast<const f32x4*>(a.taps + (size_t)(ch + e) * 4));
+  if (m0 == 0) {   // rows before the group: columns 1 .. 3 of the state
 #pragma unroll
-    for (int e = 0; e < 4; ++e) tap[e] = *as_global(reinterpret_cast<const f32x4*>(a.taps + (size_t)(ch + e) * 4));
-    if (m0 < 3) {   // rows before the group: columns 1 .. 3 of the state (row -i in column 4 - i)
-      f32x4 st[4];
+    for (int e = 0; e < 4; ++e) {
+      const f32x4 st = *as_global(reinterpret_cast<const f32x4*>(a.state + (size_t)(ch + e) * 4));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) st[e] = *as_global(reinterpret_cast<const f32x4*>(a.state + (size_t)(ch + e) * 4));
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const int m = m0 - 3 + i;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) in[i][e] = m == -3 ? st[e][1] : m == -2 ? st[e][2] : st[e][3];
-        if (m >= 0) in[i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)m * 8192 + ch));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 3; ++i) in[i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)(m0 - 3 + i) * 8192 + ch));
+      for (int i = 0; i < 3; ++i) in[i][e] = st[1 + i];
     }
+  } else {
 #pragma unroll
-    for (int i = 0; i < kConvTok; ++i)
-      in[3 + i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)min(m0 + i, a.M - 1) * 8192 + ch));
+    for (int i = 0; i < 3; ++i) in[i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)(m0 - 3 + i) * 8192 + ch));
+  }
 #pragma unroll
-    for (int k = 0; k < kConvTok; ++k) {
-      f32x4 x;
+  for (int i = 0; i < kConvTok; ++i)
+    in[3 + i] = *as_global(reinterpret_cast<const f32x4*>(a.y + (size_t)min(m0 + i, a.M - 1) * 8192 + ch));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float acc = 0.0f;
+  for (int k = 0; k < kConvTok; ++k) {
+    f32x4 x;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc = acc + in[k + i][e] * tap[e][i];
-        x[e] = dev_silu(acc);
-      }
-      *as_lds_w(reinterpret_cast<f32x4*>(xl + k * QH_CONV_DIM + ch)) = x;
+    for (int e = 0; e < 4; ++e) {
+      float acc = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc = acc + in[k + i][e] * tap[e][i];
+      x[e] = dev_silu(acc);
     }
+    *as_lds_w(reinterpret_cast<f32x4*>(xl + k * kConvCh + 4 * t)) = x;
   }
   lds_barrier();
-  const int c = t, part = c >> 7, h = (c & 127) >> 3, kg = c & 7;   // q, k or v; head; k-group
-#pragma unroll 1
-  for (int k = 0; k < kConvTok; ++k) {
-    const int m = m0 + k;
-    if (m >= a.M) break;
-    float x[16];
-    load16l(xl + k * QH_CONV_DIM + 16 * c, x);
-    if (part < 2) {   // deltanet.hpp:134,166-169 (whole waves: c / 128 is wave-uniform)
-      float ss = dot16_f32(x, x, 0.0f);
-      ss = xor_sum<8>(ss);
-      const float inv = 1.0f / sqrtf(ss + 1e-6f);
+  const int part = (int)blockIdx.y >> 2, c = 32 * ((int)blockIdx.y & 3) + (t & 31);   // q, k or v; chunk of its 128
+  const int h = c >> 3, kg = c & 7, m = m0 + (t >> 5);
+  float x[16];
+  load16l(xl + 16 * t, x);   // (token t / 32, chunk t % 32)
+  if (part < 2) {   // deltanet.hpp:134,166-169
+    float ss = dot16_f32(x, x, 0.0f);
+    ss = xor_sum<8>(ss);
+    const float inv = 1.0f / sqrtf(ss + 1e-6f);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) x[e] = x[e] * inv;
-      if (part == 0) {
-        const float sc = 1.0f / sqrtf(128.0f);
+    for (int e = 0; e < 16; ++e) x[e] = x[e] * inv;
+    if (part == 0) {
+      const float sc = 1.0f / sqrtf(128.0f);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) x[e] = x[e] * sc;
-      }
-      float* p = a.qk + ((size_t)h * a.M + m) * 256 + 128 * part + 8 * kg;
-#pragma unroll
-      for (int d = 0; d < 4; ++d)   // half d / 2, quad d % 2
-        *as_global_w(reinterpret_cast<f32x4*>(p + 64 * (d & 1) + 4 * (d >> 1))) =
-            f32x4{x[4 * d], x[4 * d + 1], x[4 * d + 2], x[4 * d + 3]};
-    } else {
-      float* p = a.v + ((size_t)h * a.M + m) * 128 + 16 * kg;
-#pragma unroll
-      for (int d = 0; d < 4; ++d)
-        *as_global_w(reinterpret_cast<f32x4*>(p + 4 * d)) = f32x4{x[4 * d], x[4 * d + 1], x[4 * d + 2], x[4 * d + 3]};
+      for (int e = 0; e < 16; ++e) x[e] = x[e] * sc;
     }
+    if (m >= a.M) return;
+    float* p = a.qk + ((size_t)h * a.M + m) * 256 + 128 * part + 8 * kg;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)   // half d / 2, quad d % 2
+      *as_global_w(reinterpret_cast<f32x4*>(p + 64 * (d & 1) + 4 * (d >> 1))) =
+          f32x4{x[4 * d], x[4 * d + 1], x[4 * d + 2], x[4 * d + 3]};
+  } else if (m < a.M) {
+    float* p = a.v + ((size_t)h * a.M + m) * 128 + 16 * kg;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      *as_global_w(reinterpret_cast<f32x4*>(p + 4 * d)) = f32x4{x[4 * d], x[4 * d + 1], x[4 * d + 2], x[4 * d + 3]};
   }
 }
 
@@ -1076,7 +1068,7 @@ hipError_t pf_gemm(const PfGemm& a, int K, PfEpi epi, int mode, hipStream_t s) {
 }
 
 hipError_t pf_conv(const PfConv& a, hipStream_t s) {
-  pf_conv_kernel<<<(a.M + kConvTok - 1) / kConvTok, 384, 0, s>>>(a);
+  pf_conv_kernel<<<dim3((a.M + kConvTok - 1) / kConvTok, QH_CONV_DIM / kConvCh), 128, 0, s>>>(a);
   return hipGetLastError();
 }
 hipError_t pf_scan(const PfScan& a, hipStream_t s) {
