@@ -519,6 +519,10 @@ __device__ __forceinline__ float pair_even(float v) {
 __device__ __forceinline__ float pair_odd(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xF5, 0xF, 0xF, false));   // quad_perm [1,1,3,3]
 }
+template <int N>   // the value N lanes away, round the row of 16
+__device__ __forceinline__ float row_ror(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xF, 0xF, false));
+}
 // sum over i of a[i] b[i] over the pair's 16 elements in order, then over the eight k-groups: valid in odd lanes
 __device__ __forceinline__ float scan_dot(const float (&a)[8], const float (&b)[8]) {
   float t[8];
@@ -530,9 +534,11 @@ __device__ __forceinline__ float scan_dot(const float (&a)[8], const float (&b)[
   p = pair_even(p);
 #pragma unroll
   for (int i = 0; i < 8; ++i) p = p + t[i];
-  p = p + xor_perm<8>(p);   // k-groups 4, 2, 1 apart
-  p = p + xor_perm<4>(p);
-  p = p + xor_perm<2>(p);
+  // k-groups 4, 2, 1 apart: after the sum over distance 8 the values repeat every 8 lanes of the row, so
+  // that a rotation by 4 (then 2) reads the partner, in the add itself
+  p = p + row_ror<8>(p);
+  p = p + row_ror<4>(p);
+  p = p + row_ror<2>(p);
   return p;
 }
 __global__ __launch_bounds__(256, 1) void pf_scan_kernel(const PfScan a) {
@@ -578,46 +584,60 @@ __global__ __launch_bounds__(256, 1) void pf_scan_kernel(const PfScan a) {
       o[4 + e] = y[e];
     }
   };
-  // n tokens of block b (FULL: all eight, straight-line)
+  // n tokens of block b (FULL: all eight, straight-line).  Token t + 2's vectors are read while token t
+  // runs (the empty asm keeps the reads above it: next to their use, each token waited for the LDS; 768
+  // tokens took 157.7 us, with the reads ahead 146.1, and with the tree's rotations 143.1).
   auto runA = [&](int b, auto full, int n) {
     const ScanBlock& B = blk[b % 3];
     float* d_out = dl[b & 1] + 32 * half;
     const float cg = as_lds(B.g)[lane & 15];
+    float k[3][8], vt[3];
+    auto get = [&](int t) {
+      ld8(B.qk + 256 * t + 128, k[t % 3]);
+      vt[t % 3] = as_lds(B.v)[8 * t + 4 * half + vc];
+    };
+    get(0);
+    get(1);
 #pragma unroll
     for (int t = 0; t < kScanTok; ++t) {
       if (!decltype(full)::value && t >= n) break;
-      float k[8];
-      ld8(B.qk + 256 * t + 128, k);
-      const float vt = as_lds(B.v)[8 * t + 4 * half + vc];
+      if (t + 2 < kScanTok) get(t + 2);
+      asm volatile("" ::: "memory");
+      const float (&kt)[8] = k[t % 3];
       const float gexp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t));
       const float beta = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t + 1));
 #pragma unroll
       for (int i = 0; i < 8; ++i) s[i] = s[i] * gexp;
-      const float d = pair_odd((vt - scan_dot(s, k)) * beta);
+      const float d = pair_odd((vt[t % 3] - scan_dot(s, kt)) * beta);
       if (kh == 0) as_lds_w(d_out)[4 * t + vc] = d;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) s[i] = s[i] + k[i] * d;
+      for (int i = 0; i < 8; ++i) s[i] = s[i] + kt[i] * d;
     }
   };
   auto runB = [&](int b, auto full, int n) {
     const ScanBlock& B = blk[b % 3];
     const float* d_in = dl[b & 1] + 32 * half;
     const float cg = as_lds(B.g)[lane & 15];
-    float ov = 0.0f;
+    float ov = 0.0f, k[3][8], q[3][8], d[3];
+    auto get = [&](int t) {
+      ld8(B.qk + 256 * t + 128, k[t % 3]);
+      ld8(B.qk + 256 * t, q[t % 3]);
+      d[t % 3] = as_lds(d_in)[4 * t + vc];
+    };
+    get(0);
+    get(1);
 #pragma unroll
     for (int t = 0; t < kScanTok; ++t) {
       if (!decltype(full)::value && t >= n) break;
-      float k[8], q[8];
-      ld8(B.qk + 256 * t + 128, k);
-      ld8(B.qk + 256 * t, q);
-      const float d = as_lds(d_in)[4 * t + vc];
+      if (t + 2 < kScanTok) get(t + 2);
+      asm volatile("" ::: "memory");
       const float gexp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cg), 2 * t));
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         s[i] = s[i] * gexp;
-        s[i] = s[i] + k[i] * d;
+        s[i] = s[i] + k[t % 3][i] * d[t % 3];
       }
-      const float p = scan_dot(s, q);
+      const float p = scan_dot(s, q[t % 3]);
       if (kg == t) ov = p;
     }
     if ((lane & 1) && kg < n) as_global_w(a.o)[(size_t)(b * kScanTok + kg) * 2048 + h * 128 + v] = ov;
