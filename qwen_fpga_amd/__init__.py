@@ -93,9 +93,9 @@ def _lib() -> ctypes.CDLL:
         # runtime beside /opt/rocm's, and the one initialised second sees no
         # device.  So when torch is importable it is loaded before libqh.
         try:
-            import torch  # noqa: F401
+            import torch
         except ImportError:
-            pass
+            torch = None
         lib = ctypes.CDLL(LIB_PATH)
         lib.qh_strerror.restype = ctypes.c_char_p
         lib.qh_blob_size.restype = ctypes.c_size_t
@@ -112,6 +112,11 @@ def _lib() -> ctypes.CDLL:
         lib.qh_engine_last_launch_ms.argtypes = [ctypes.c_void_p]
         lib.qh_engine_device_ptr.restype = ctypes.c_void_p
         lib.qh_engine_device_ptr.argtypes = [ctypes.c_void_p, ctypes.c_int]
+        if torch is not None:   # (not at the package's import, which host-only users of the layout and packer share)
+            _Short.f32, _Short.i8, _Short.i32 = torch.float32, torch.int8, torch.int32
+            _Short.device = getattr(torch._C, "_cuda_getDevice", None)
+            _Short.stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+            _Short.tensor = torch.Tensor
         _LIB = lib
     return _LIB
 
@@ -250,18 +255,8 @@ def _op(name: str):
 
 
 class _Short:
-    """torch's tensor class, dtypes and raw stream query, looked up once (torch may be absent)."""
+    """torch's tensor class, dtypes and raw stream query, looked up once by _lib (torch may be absent)."""
     tensor = f32 = i8 = i32 = device = stream = None
-
-
-try:
-    import torch as _torch
-
-    _Short.tensor, _Short.f32, _Short.i8, _Short.i32 = _torch.Tensor, _torch.float32, _torch.int8, _torch.int32
-    _Short.device = getattr(_torch._C, "_cuda_getDevice", None)
-    _Short.stream = getattr(_torch._C, "_cuda_getCurrentRawStream", None)
-except ImportError:
-    pass
 
 
 def _slow(t, kind: str, n: int, what: str) -> Optional[int]:

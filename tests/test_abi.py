@@ -3,6 +3,7 @@ arguments on the host (CPU; nothing here launches device work)."""
 import ctypes
 import os
 import subprocess
+import sys
 
 import pytest
 
@@ -69,3 +70,16 @@ def test_run_hls_cli_usage_and_missing_blob(tmp_path):
     empty.write_text("")
     r = subprocess.run([exe, str(tmp_path / "missing.bin"), str(empty), "4"], capture_output=True, text=True)
     assert r.returncode == 2 and "no prompt ids" in r.stderr
+
+
+def test_import_leaves_torch_alone():
+    """The package and its host-only users (layout index, packer) import without torch; it is loaded
+    with the library, on first use, and the ops' short argument checks are in place from then on."""
+    code = ("import sys\n"
+            "import qwen_fpga_amd as q, qwen_fpga_amd.pack_weights\n"
+            "assert 'torch' not in sys.modules and q._Short.tensor is None\n"
+            "q._lib()\n"
+            "import torch\n"
+            "assert q._Short.tensor is torch.Tensor and q._Short.f32 is torch.float32\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
+    assert r.returncode == 0, r.stderr
