@@ -51,7 +51,9 @@ extern "C" {
                             QH_TAG_START, starts the persistent kernel's hand-over tags
                             at that value instead of 1, so that a test reaches the
                             launch that would run past 2^32 - 1 (the engine then
-                            clears the tagged buffers and restarts the tags at 1). */
+                            clears the tagged buffers and restarts the tags at 1).  A
+                            third, QH_FAIL_SETUP=prepare|launch, fails one set-up step of
+                            an executor once (QH_ENOMEM). */
 
 /* ---- model dimensions (hls/src/types.hpp:20-44) ----------------------- */
 #define QH_HIDDEN 1024
@@ -279,7 +281,10 @@ int qh_decode_token(qh_engine* e, int tok, float* logits, int* argmax_out);
  * feedback stays on the device: one persistent launch (or one graph replay per
  * token) and no host round trip between tokens.  A prompt's tokens but the last
  * run in groups (one read of the weights per group of up to 512 tokens) where
- * that is faster; the state they leave is the token-by-token state bit for bit. */
+ * that is faster; the state they leave is the token-by-token state bit for bit.
+ * An error while or after they run leaves an engine that refuses to decode
+ * (QH_ESTATE) until qh_engine_reset; an earlier one leaves state and position
+ * as they were. */
 int qh_generate(qh_engine* e, const int* prompt, int n_prompt, int n_new, int eos, int* out_ids,
                 int* n_out);
 /* Tokens processed so far (DecodeState::pos). */

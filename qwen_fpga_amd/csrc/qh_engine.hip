@@ -81,7 +81,8 @@ struct qh_engine {
   hipEvent_t launch_ev[2] = {};  // around the last persistent launch (engine stream)
   float last_launch_ms = 0.0f;
   unsigned poll_limit = 1u << 20;  // failed polls before a hand-over wait gives up (QH_POLL_LIMIT)
-  bool broken = false;             // a launch returned QH_EDEVICE: decode refused until reset
+  bool broken = false;             // a call ended with the state between two tokens': decode refused until reset
+  int fail_setup = 0;              // test hook QH_FAIL_SETUP: the set-up step that fails (FAIL_*), once
   int fallbacks = 0;               // cooperative launches refused (each switched the engine to the graph path)
   // Grouped prompt path (qh_prefill.hip), made by the first prompt that takes it: the buffers of
   // up to kPfSlots groups, a stream for each slot after the first (which runs on `stream`), and
@@ -455,10 +456,19 @@ int enqueue_layers(qh_engine* e, int l0, int l1, bool embed, hipStream_t s) {
   return launch_stages(e, v, s);
 }
 
+// Test hook: true the first time the chosen set-up step is reached.
+enum { FAIL_PREPARE = 1, FAIL_LAUNCH = 2 };   // making the program or graph; the launch that uses it
+bool setup_fails(qh_engine* e, int step) {
+  if (e->fail_setup != step) return false;
+  e->fail_setup = 0;
+  return true;
+}
+
 // The persistent kernel's per-token program for the current mode, over the
 // tagged arena (allocated and zeroed on first use; both modes share it).
 int ensure_prog(qh_engine* e) {
   if (e->prog[e->mode]) return QH_OK;
+  if (setup_fails(e, FAIL_PREPARE)) return QH_ENOMEM;
   std::vector<Stage> v;
   Vec h;
   if (e->arena == nullptr) {
@@ -520,6 +530,7 @@ constexpr int kUseGraph = 1000;
 int run_persist(qh_engine* e, int tok0, int step0, int n_prompt, int n_new, int eos, bool with_logits, bool set_prompt,
                 StepCtl* out) {
   QH_TRY(ensure_prog(e));
+  if (setup_fails(e, FAIL_LAUNCH)) return QH_ENOMEM;
   hipStream_t s = e->stream;
   // tags of this launch: tag_base + k * kTagsPerToken + stage, k < n_prompt - step0 + n_new
   const uint64_t need = ((uint64_t)(n_prompt - step0) + (uint64_t)n_new + 1) * kTagsPerToken;
@@ -633,6 +644,7 @@ int enqueue_step(qh_engine* e, bool with_logits, bool advance, hipStream_t s,
 int get_graph(qh_engine* e, bool with_logits, bool advance, hipGraphExec_t* out) {
   hipGraphExec_t& ge = e->graphs[e->mode][with_logits][advance];
   if (ge == nullptr) {
+    if (setup_fails(e, FAIL_PREPARE)) return QH_ENOMEM;
     hipGraph_t g = nullptr;
     QH_HIP(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
     const int st = enqueue_step(e, with_logits, advance, e->stream);
@@ -906,6 +918,38 @@ int run_prefill(qh_engine* e, int n, int* done) {
   return QH_OK;
 }
 
+// The rest of a qh_generate call on the executor: prompt tokens step0 .. and the new ones.
+int run_rest(qh_engine* e, const int* prompt, int step0, int n_prompt, int n_new, int eos, int* out_ids, int* n_out) {
+  if (e->exec == QH_EXEC_PERSISTENT) {
+    StepCtl c;
+    const int st = run_persist(e, prompt[step0], step0, n_prompt, n_new, eos, false, false, &c);
+    if (st != kUseGraph) {
+      QH_TRY(st);
+      if (c.n_out > 0)
+        QH_HIP(hipMemcpy(out_ids, e->out_dev, sizeof(int) * (size_t)c.n_out, hipMemcpyDeviceToHost));
+      *n_out = c.n_out;
+      return c.err == 2 ? QH_ERANGE : QH_OK;
+    }
+  }
+  hipStream_t s = e->stream;
+  hipGraphExec_t g;
+  QH_TRY(get_graph(e, false, true, &g));
+  if (setup_fails(e, FAIL_LAUNCH)) return QH_ENOMEM;
+  if (step0 > 0) QH_HIP(launch_set_int(&e->ctl->pos, e->host_pos, s));
+  QH_HIP(launch_init_gen(e->ctl, prompt[step0], step0, n_prompt, n_new, eos, s));
+  for (int i = step0; i < n_prompt + n_new; ++i) QH_HIP(hipGraphLaunch(g, s));
+  StepCtl c;
+  QH_HIP(hipMemcpyAsync(&c, e->ctl, sizeof c, hipMemcpyDeviceToHost, s));
+  QH_HIP(hipStreamSynchronize(s));
+  if (c.n_out > 0) QH_HIP(hipMemcpy(out_ids, e->out_dev, sizeof(int) * (size_t)c.n_out, hipMemcpyDeviceToHost));
+  *n_out = c.n_out;
+  e->host_pos = c.pos;
+  e->last_argmax = c.argmax;
+  QH_HIP(launch_set_int(&e->ctl->done, 0, s));
+  QH_HIP(hipStreamSynchronize(s));
+  return c.err == 2 ? QH_ERANGE : QH_OK;
+}
+
 void release(qh_engine* e) {
   if (!e) return;
   if (e->stream) (void)hipStreamSynchronize(e->stream);
@@ -1001,6 +1045,8 @@ int create(const void* blob, size_t blob_len, const char* idx_text, int max_ctx,
     const unsigned long long v = std::strtoull(ts, nullptr, 10);
     if (v >= 1 && v <= 0xFFFFFFFFull) e->tag_start = (uint32_t)v;
   }
+  if (const char* fs = std::getenv("QH_FAIL_SETUP"))   // test hook: an executor's set-up fails, once
+    e->fail_setup = std::strcmp(fs, "prepare") == 0 ? FAIL_PREPARE : std::strcmp(fs, "launch") == 0 ? FAIL_LAUNCH : 0;
   e->nsplit_max = attn_nsplit_max(max_ctx);
   e->head_grid = kVocab / (kRowsPerBatch * 4 * 4);   // 4 waves x 4 batches per block
   int st = QH_OK;
@@ -1185,37 +1231,19 @@ int qh_generate(qh_engine* e, const int* prompt, int n_prompt, int n_new, int eo
     if (prompt[i] < 0 || prompt[i] >= kVocab) return QH_ERANGE;
   if ((long)e->host_pos + n_prompt + n_new > e->max_ctx) return QH_ERANGE;
   QH_TRY(ensure_io(e, n_prompt > n_new ? n_prompt : n_new));
+  // the executor's program or graph before the groups: its failure leaves state and position alone
+  hipGraphExec_t g;
+  QH_TRY(e->exec == QH_EXEC_PERSISTENT ? ensure_prog(e) : get_graph(e, false, true, &g));
   hipStream_t s = e->stream;
   QH_HIP(hipMemcpyAsync(e->prompt_dev, prompt, sizeof(int) * (size_t)n_prompt, hipMemcpyHostToDevice, s));
   QH_HIP(hipStreamSynchronize(s));
   int step0 = 0;   // prompt tokens run as groups; the rest, the last one at least, one by one
   QH_TRY(run_prefill(e, prefill_tokens(e, n_prompt), &step0));
-  if (e->exec == QH_EXEC_PERSISTENT) {
-    StepCtl c;
-    const int st = run_persist(e, prompt[step0], step0, n_prompt, n_new, eos, false, false, &c);
-    if (st != kUseGraph) {
-      QH_TRY(st);
-      if (c.n_out > 0)
-        QH_HIP(hipMemcpy(out_ids, e->out_dev, sizeof(int) * (size_t)c.n_out, hipMemcpyDeviceToHost));
-      *n_out = c.n_out;
-      return c.err == 2 ? QH_ERANGE : QH_OK;
-    }
-  }
-  hipGraphExec_t g;
-  QH_TRY(get_graph(e, false, true, &g));
-  if (step0 > 0) QH_HIP(launch_set_int(&e->ctl->pos, e->host_pos, s));
-  QH_HIP(launch_init_gen(e->ctl, prompt[step0], step0, n_prompt, n_new, eos, s));
-  for (int i = step0; i < n_prompt + n_new; ++i) QH_HIP(hipGraphLaunch(g, s));
-  StepCtl c;
-  QH_HIP(hipMemcpyAsync(&c, e->ctl, sizeof c, hipMemcpyDeviceToHost, s));
-  QH_HIP(hipStreamSynchronize(s));
-  if (c.n_out > 0) QH_HIP(hipMemcpy(out_ids, e->out_dev, sizeof(int) * (size_t)c.n_out, hipMemcpyDeviceToHost));
-  *n_out = c.n_out;
-  e->host_pos = c.pos;
-  e->last_argmax = c.argmax;
-  QH_HIP(launch_set_int(&e->ctl->done, 0, s));
-  QH_HIP(hipStreamSynchronize(s));
-  return c.err == 2 ? QH_ERANGE : QH_OK;
+  const int st = run_rest(e, prompt, step0, n_prompt, n_new, eos, out_ids, n_out);
+  // Groups that ran have advanced the state past the executor's position: a failure after them ends
+  // between two states.  (QH_ERANGE is the executor's own end at the context's limit.)
+  if (step0 > 0 && st != QH_OK && st != QH_ERANGE) e->broken = true;
+  return st;
 }
 
 int qh_engine_pos(const qh_engine* e) { return e ? e->host_pos : -1; }

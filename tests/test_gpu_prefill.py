@@ -88,3 +88,38 @@ def test_generation_after_a_grouped_prompt(q, blob, torch_cuda):
             assert e.generate(ids, 12, eos=want[5]) == want[:first] and e.pos == 70 + first
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("exec_kind", ["graph", "persistent"])
+@pytest.mark.parametrize("step", ["prepare", "launch"])
+def test_setup_failure_around_the_groups(q, blob, torch_cuda, monkeypatch, exec_kind, step):
+    """An executor whose set-up fails (forced from the host: QH_FAIL_SETUP) while a prompt runs in
+    groups.  The program or graph is made first, so that its failure leaves position and state as they
+    were and the same call then succeeds; a failure after the groups leaves an engine that refuses to
+    decode until its reset.  Both end with what an engine without the failure gives."""
+    monkeypatch.setenv("QH_FAIL_SETUP", step)
+    e = q.Engine(blob, max_ctx=64)
+    monkeypatch.delenv("QH_FAIL_SETUP")
+    f = q.Engine(blob, max_ctx=64)
+    try:
+        for eng in (e, f):
+            eng.set_exec(q.EXEC_GRAPH if exec_kind == "graph" else q.EXEC_PERSISTENT)
+        ids = rng(21).integers(0, q.VOCAB, size=20).astype(np.int32).tolist()
+        want, lw = f.generate(ids, 4), f.decode_token(7, want_logits=True)[1]
+        with pytest.raises(q.QHError) as ex:
+            e.generate(ids, 4)
+        assert ex.value.status == q.QH_ENOMEM
+        if step == "prepare":
+            assert e.pos == 0
+            assert all(not a.any() for a in _state(e, 64, 64)), "state touched by the failed call"
+        else:
+            for call in (lambda: e.decode_token(7), lambda: e.generate(ids, 4)):
+                with pytest.raises(q.QHError) as ex:
+                    call()
+                assert ex.value.status == q.QH_ESTATE
+            e.reset()
+        assert e.generate(ids, 4) == want and e.pos == 24
+        assert_bitwise(e.decode_token(7, want_logits=True)[1], lw, "next logits")
+    finally:
+        e.close()
+        f.close()
