@@ -865,10 +865,12 @@ int prefill_slot(qh_engine* e, int i, int G, bool events) {
     e->pf_cap[i] = cap;
   }
   if (e->pf_stream[i] == nullptr) {
-    if (i == 0)
+    if (i == 0) {
+      QH_HIP(pf_attn_setup());
       e->pf_stream[i] = e->stream;
-    else
+    } else {
       QH_HIP(hipStreamCreate(&e->pf_stream[i]));
+    }
   }
   if (events)
     for (hipEvent_t& ev : e->pf_ev[i])

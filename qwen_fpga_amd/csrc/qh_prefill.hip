@@ -1116,15 +1116,25 @@ hipError_t pf_qk(const PfAttn& a, hipStream_t s) {
   pf_qk_kernel<<<a.M + (a.pos0 + 7) / 8, 256, 0, s>>>(a);
   return hipGetLastError();
 }
+namespace {
+constexpr int pf_attn_lds(int last) {   // bytes of a launch whose last cache row is `last` (pf_attn_kernel's dyn)
+  return (int)sizeof(float) * (16 * (16 * ((last >> 4) + 1) + 4) + 2 * 16 * ((last >> 4) + 3) + 16);
+}
+}  // namespace
+// The launches' limit is a property of the kernel, shared by every engine and thread of the process: it
+// is set once, to the largest size, and never lowered between another thread's check and its launch.
+hipError_t pf_attn_setup() {
+  constexpr int lds = pf_attn_lds(kPfMaxPos - 1);
+  static_assert(lds <= 160 * 1024, "one workgroup's LDS");
+  for (const void* fn : {reinterpret_cast<const void*>(pf_attn_kernel<M_W8A8>), reinterpret_cast<const void*>(pf_attn_kernel<M_W8A16>)})
+    if (const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds); e != hipSuccess) return e;
+  return hipSuccess;
+}
 hipError_t pf_attn(const PfAttn& a, int mode, hipStream_t s) {
   const int last = a.pos0 + a.M - 1;
   if (a.M < 1 || last >= kPfMaxPos) return hipErrorInvalidValue;
   const int tiles = (last >> 4) - (a.pos0 >> 4) + 1;
-  const size_t lds = sizeof(float) * (16 * (16 * ((last >> 4) + 1) + 4) + 2 * 16 * ((last >> 4) + 3) + 16);
-  const void* fn = mode == M_W8A8 ? reinterpret_cast<const void*>(pf_attn_kernel<M_W8A8>)
-                                  : reinterpret_cast<const void*>(pf_attn_kernel<M_W8A16>);
-  if (const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); e != hipSuccess)
-    return e;
+  const size_t lds = pf_attn_lds(last);
   if (mode == M_W8A8)
     pf_attn_kernel<M_W8A8><<<8 * tiles, 256, lds, s>>>(a);
   else

@@ -121,6 +121,8 @@ hipError_t pf_conv(const PfConv& a, hipStream_t s);
 hipError_t pf_scan(const PfScan& a, hipStream_t s);
 hipError_t pf_gated(const PfGated& a, int mode, hipStream_t s);
 hipError_t pf_qk(const PfAttn& a, hipStream_t s);
+// once per engine, before its first pf_attn: the kernels' dynamic LDS limit
+hipError_t pf_attn_setup();
 hipError_t pf_attn(const PfAttn& a, int mode, hipStream_t s);
 // rows of x [M][K] quantised into fragments (W8A8), K = 2048 or 3584
 hipError_t pf_quant(void* xf, float* xs, const float* x, int K, int M, hipStream_t s);

@@ -3,6 +3,8 @@ bit: the recurrent, conv and KV state, the next token and its logits.  Lengths a
 MFMA tiles (16 and 32 tokens) and of the scan's blocks (8), of one group (512, then two halves), of
 the positions the grouped attention covers (2048), and prompts that start inside a tile.  The prompt's last token always runs on the executor, so n
 tokens take the grouped path for n - 1 of them."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -123,3 +125,38 @@ def test_setup_failure_around_the_groups(q, blob, torch_cuda, monkeypatch, exec_
     finally:
         e.close()
         f.close()
+
+
+def test_two_engines_prompt_in_two_threads(q, blob, torch_cuda):
+    """A short and a long prompt, whose attention launches need 4 and 68 KiB of LDS, in two threads at
+    once: each engine's state is what it is alone (the kernel's LDS limit belongs to the process)."""
+    r = rng(31)
+    prompts = [r.integers(0, q.VOCAB, size=n).astype(np.int32).tolist() for n in (40, 950)]
+    es = [q.Engine(blob, max_ctx=len(p) + 4, mode=q.MODE_W8A8) for p in prompts]
+    try:
+        want = []
+        for e, p in zip(es, prompts):
+            e.set_exec(q.EXEC_GRAPH)
+            gen = e.generate(p, 2)
+            want.append((gen, _state(e, len(p), len(p) + 4)))
+        got = [[], []]
+        start = threading.Barrier(2)
+
+        def work(i, passes):
+            start.wait()
+            for _ in range(passes):
+                es[i].reset()
+                got[i].append(es[i].generate(prompts[i], 2))
+
+        ts = [threading.Thread(target=work, args=a) for a in ((0, 12), (1, 4))]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        for i, (e, p) in enumerate(zip(es, prompts)):
+            assert got[i] and all(g == want[i][0] for g in got[i])
+            for a, b, what in zip(_state(e, len(p), len(p) + 4), want[i][1], ("recurrent state", "conv state", "k cache", "v cache")):
+                assert_bitwise(a, b, f"{what}, prompt of {len(p)}")
+    finally:
+        for e in es:
+            e.close()
