@@ -691,20 +691,35 @@ struct PfBufs {
   }
 };
 
-// The shortest run of prompt tokens that goes as a group.  A group takes 1.6 ms in W8A8 and 2.6 ms in
-// W8A16 at 4 to 32 tokens (240 launches, every weight byte read once); a token by itself takes 0.42 ms
-// on the persistent executor and 0.75 ms on the graph executor.
-int prefill_min(const qh_engine* e) {
-  if (e->exec == QH_EXEC_PERSISTENT) return e->mode == M_W8A8 ? 5 : 7;
-  return e->mode == M_W8A8 ? 3 : 4;
+// The shortest run of prompt tokens, starting at position pos, that goes as a group.  Measured with the
+// prompt's last token on the executor, groups / token by token, ms:
+//   executor    mode   tokens   pos 0      1000        1500        1850
+//   persistent  W8A8     5    2.03/2.68  2.71/3.02   3.05/3.17   3.27/3.25
+//                        6    2.08/3.13  2.68/3.48   2.98/3.66   3.24/3.75
+//   persistent  W8A16    6    3.01/3.16  3.62/3.52   3.93/3.67   4.17/3.78
+//                        7    3.07/3.62  3.67/4.04   4.01/4.20   4.24/4.31
+//   graph       W8A8     3    2.12/3.03  2.74/3.16   3.05/3.19   3.27/3.24
+//                        4    2.15/3.77  2.79/3.93   3.09/3.99   3.29/4.02
+//   graph       W8A16    4    3.05/3.55  3.67/3.70   3.97/3.77   4.17/3.79
+//                        5    3.05/4.25  3.66/4.43   3.98/4.52   4.18/4.55
+// A group is launches (240 in W8A8, 210 in W8A16) and one read of the weights, whatever its size; the
+// older keys' fragments and the attention, whose workgroups walk all earlier positions, add 0.6 ms per
+// 1000 positions, where a token by itself takes 0.05 ms more.
+constexpr int prefill_min(bool persistent, bool w8a8, int pos) {
+  if (persistent) return w8a8 ? (pos <= 1500 ? 5 : 6) : 7;
+  return w8a8 ? (pos <= 1500 ? 3 : 4) : (pos <= 1000 ? 4 : 5);
 }
+static_assert(prefill_min(true, true, 0) == 5 && prefill_min(true, true, 1850) == 6 && prefill_min(true, false, 1850) == 7 &&
+                  prefill_min(false, true, 0) == 3 && prefill_min(false, true, 1850) == 4 &&
+                  prefill_min(false, false, 0) == 4 && prefill_min(false, false, 1500) == 5,
+              "no group where token by token is faster");
 
 // How many of a prompt's first tokens run in groups: all but the last (the executor runs it, with the
 // LM head), up to the positions the grouped attention covers.
 int prefill_tokens(const qh_engine* e, int n_prompt) {
   int n = n_prompt - 1;
   if (n > kPfMaxPos - e->host_pos) n = kPfMaxPos - e->host_pos;
-  return n < prefill_min(e) || e->pf_off ? 0 : n;
+  return n < prefill_min(e->exec == QH_EXEC_PERSISTENT, e->mode == M_W8A8, e->host_pos) || e->pf_off ? 0 : n;
 }
 
 // Tokens per group of a prompt of n (at most kPfMaxPos): one group up to 512 tokens, above that two

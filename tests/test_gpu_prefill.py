@@ -68,6 +68,25 @@ def test_prompt_past_the_short_contexts(q, blob, torch_cuda, mode):
         e.close()
 
 
+# the shortest groups that the rule takes (prefill_min) at the start of a context and late in one
+@pytest.mark.parametrize("mode,exec_kind,first,late", [(0, "graph", 4, 5), (1, "graph", 3, 4), (0, "persistent", 7, 7),
+                                                       (1, "persistent", 5, 6)])
+def test_shortest_groups(q, blob, torch_cuda, mode, exec_kind, first, late):
+    """Both sides of the rule's line, from an empty state and after other prompts (a group shorter than
+    the four conv taps keeps an old column, and the scan's only block is partial)."""
+    ctx = 1900
+    e = q.Engine(blob, max_ctx=ctx, mode=mode)
+    try:
+        e.set_exec(q.EXEC_GRAPH if exec_kind == "graph" else q.EXEC_PERSISTENT)
+        r = rng(55 + mode)
+        ids = lambda n: r.integers(0, q.VOCAB, size=n).astype(np.int32).tolist()
+        for ls in ([first + 1], [first], [2, first + 1, first + 2], [first + 1, 1, first, first + 1],
+                   [1842, late + 1, late, first + 1]):
+            _check(q, e, [ids(n) for n in ls], ctx)
+    finally:
+        e.close()
+
+
 def test_generation_after_a_grouped_prompt(q, blob, torch_cuda):
     """Greedy ids, eos and the position after a grouped prompt equal those of a host loop."""
     ctx = 128
