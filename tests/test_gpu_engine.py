@@ -7,8 +7,8 @@
   compiled hls/src kernels): identical argmax at every one of 576 steps;
 * the run_hls generation loop (hls/tb/run_hls.cpp:56-66) on the device against
   a host loop of decode_token calls, eos handling, context limits, reset;
-* the benchmarked configuration (persistent executor, W8A8, 64 + 512 tokens in
-  one launch) bit for bit against the twin; the argmax tie rule across
+* the benchmarked configuration (persistent executor, W8A8, a prompt of 64 and
+  512 tokens in one call) bit for bit against the twin; the argmax tie rule across
   workgroups; a forced hand-over give-up that every wave survives;
 * layers [0, 4) as one block for 128 steps (C4), and the qh_run_hls CLI.
 """
@@ -213,10 +213,10 @@ def test_forward_layers_block_c4(q, orc, blob, idx, torch_cuda, mode):
 
 def test_persistent_full_c5_w8a8_vs_twin(q, orc, blob, idx, torch_cuda):
     """The benchmarked path at the benchmarked length: the persistent executor, W8A8, the C5
-    prompt (64 seeded ids) and 512 greedy tokens in ONE launch (KV to 576, the multi-chunk
-    combine past 512 positions), against the device twin: every generated id and, at the end,
-    every recurrent / conv / KV buffer bit for bit; then the same stream token by token with
-    the logits of chosen steps bit for bit."""
+    prompt (64 seeded ids, 63 of them as a group) and 512 greedy tokens in one call (KV to 576, the
+    multi-chunk combine past 512 positions; one launch from the prompt's last token on), against the
+    device twin: every generated id and, at the end, every recurrent / conv / KV buffer bit for bit;
+    then the same stream token by token with the logits of chosen steps bit for bit."""
     npr, nn = 64, 512
     prompt = rng(1234).integers(0, q.VOCAB, size=npr).astype(np.int32).tolist()
     n = npr + nn
@@ -384,7 +384,9 @@ def test_tag_space_wrap(q, blob, torch_cuda, monkeypatch):
     and restarts the tags at 1 (qh_engine.hip run_persist).  Forced from the host by starting the
     tags just below the top (QH_TAG_START): the second of three launches wraps, and the ids,
     logits and every state buffer equal those of an engine whose tags start at 1."""
-    top = 0xFFFFFFFF - 5000   # launch 1 needs 17 * 256 = 4352 tags, launch 2 another 10 * 256
+    # Launches 1 and 2 need 10 * 256 tags each: 7 of the 8 prompt tokens run as a group, without tags; the
+    # last one, 8 new ones and one to spare.  3800 holds the first (1240 left) and not the second (1320 short).
+    top = 0xFFFFFFFF - 3800
     monkeypatch.setenv("QH_TAG_START", str(top))
     e = q.Engine(blob, max_ctx=64)
     monkeypatch.delenv("QH_TAG_START")
