@@ -3,7 +3,7 @@
 
 Workload ("C5"): the full Qwen3.5-0.8B-shaped model
 with seeded synthetic int8 weights in the packed pack_weights.py layout; a
-64-token seeded prompt is fed through the recurrent path (untimed), then
+64-token seeded prompt is fed (untimed; all but its last token as one group), then
 `--steps` greedy decode steps are timed (default 512, so the KV cache grows to
 576).  One "step" is one decode token: embed, 24 layers, final norm, the tied
 248320x1024 int8 head and its on-device argmax, run by the persistent
@@ -380,7 +380,7 @@ def op_configs(q, torch, np, blob, idx, act_mode, with_c4=True):
     us = _timed(torch, lambda i=0: q.deltanet_step(o, qkv, z, b, a, cw[i % copies], A_log, dtb, nw, S[i % copies],
                                                    cst[i % copies], ws), 200)
     out["C2_deltanet_step"] = entry("C2", 2_384_640, us, copies=copies,
-                                    ops="conv1d+SiLU+gates, l2norm+delta rule, gated RMSNorm (3 kernels)")
+                                    ops="conv1d+SiLU+gates, l2norm+delta rule, gated RMSNorm (1 kernel)")
     del S, cst, cw
 
     # C3: the gated GQA attention layer (projections, QK-norm, RoPE, split-K softmax, gate, o_proj)

@@ -278,10 +278,16 @@ int qh_decode_token(qh_engine* e, int tok, float* logits, int* argmax_out);
 /* The run_hls loop (run_hls.cpp:56-66) on the device: feed n_prompt ids, then
  * greedily generate up to n_new ids, stopping before emitting `eos` (eos < 0:
  * never).  out_ids receives the generated ids, *n_out their count.  The token
- * feedback stays on the device: one persistent launch (or one graph replay per
- * token) and no host round trip between tokens.  A prompt's tokens but the last
- * run in groups (one read of the weights per group of up to 512 tokens) where
- * that is faster; the state they leave is the token-by-token state bit for bit.
+ * feedback stays on the device: no host round trip between tokens.  A prompt's
+ * tokens but the last run in groups where there are enough of them (3 to 7, by
+ * executor, mode and position): one group up to 512 tokens, above that two of up
+ * to 1024, to position 2047; a group reads the weights once.  The remaining prompt
+ * tokens, the last one and the new ones run on the executor: one persistent launch
+ * or one graph replay per token.  The state that groups leave is the
+ * token-by-token state bit for bit.  Their buffers (18 MiB for groups of up to 128
+ * tokens, 31, 58 and 112 for 256, 512 and 1024; twice that above 512 prompt tokens)
+ * are allocated by the first prompt that needs them and kept until
+ * qh_engine_destroy; where that fails, prompts run token by token.
  * An error while or after they run leaves an engine that refuses to decode
  * (QH_ESTATE) until qh_engine_reset; an earlier one leaves state and position
  * as they were. */

@@ -723,10 +723,14 @@ int prefill_tokens(const qh_engine* e, int n_prompt) {
 }
 
 // Tokens per group of a prompt of n (at most kPfMaxPos): one group up to 512 tokens, above that two
-// halves, the second one layer behind the first on a stream of its own.  The two overlap (1024
-// tokens: 6.0 ms in W8A8 where one group after the other takes 8.4), but each is a chain of 240
-// launches: two of 256 took as long as one of 512 (4.1 ms).  A third stream made each wait between
-// groups slower by hundreds of microseconds, so there are never more than two.
+// halves, the second on a stream of its own, each of its layers after the same layer of the first.
+// Whether the halves overlap depends on the hardware queues that HIP gives the two streams, which goes
+// by the streams the process made before.  Whole prompts, ms, two halves overlapping / two halves on
+// one stream / one group: 599 tokens W8A8 4.9 / 6.6 / 5.1, W8A16 10.0 / 13.7 / 11.4; 1024 tokens W8A8
+// 6.4 / 8.7 / 7.3, W8A16 14.8 / 17.5 / 15.9; 1498 tokens W8A16 20.5 / 25.9 / -.  Where they did not
+// overlap (the second of four engines in a process, or an engine made after two other streams) 1498
+// tokens took 26.1.  With a third stream each wait between groups was slower by hundreds of
+// microseconds, so there are never more than two.
 int prefill_group_size(int n) {
   static_assert(2 * kPfGroup >= kPfMaxPos, "two groups hold every prompt");
   return n <= 512 ? n : ((n + 1) / 2 + 31) & ~31;
@@ -1075,7 +1079,8 @@ int create(const void* blob, size_t blob_len, const char* idx_text, int max_ctx,
   // The upload comes before the stream: it gives the null stream the process's first hardware queue
   // if nothing has used it yet.  The cooperative launches' queue is made last, as the fifth where a
   // process has four others, and dispatches on the queue whose pipe it shares, the first one, were
-  // 15 us slower each (a prompt's group: 6.1 instead of 2.5 ms).
+  // 15 us slower each (a prompt's group: 6.1 instead of 2.5 ms).  In a process that has used queues
+  // before, which one the stream gets is not this function's to choose.
   QH_C(dalloc(&e->blob, blob_len));
   QH_C(hip_status(hipMemcpy(e->blob, blob, blob_len, hipMemcpyHostToDevice)));
   QH_C(hip_status(hipStreamCreate(&e->stream)));

@@ -168,10 +168,20 @@ Seg seg_i8(const int8_t* w, const float* sw, int rows, int batch0, float* out, i
 
 // Rows a wave reduces together.  Eight rows share the activation's staging and reduction, but the
 // grid is rows / R waves: below one wave per SIMD (1024) the chip is idle and each wave's loads queue
-// behind one another.  Measured (us per call, R = 8 / 4 / 1): 1024x3584 W8A8 7.8 / 6.7 / 6.2, W8A16
-// 9.3 / 7.5 / 6.6; 4096x3584 W8A8 8.2 / 7.7 / 9.6; 6144x3584 W8A8 8.9 / 10.9 / 11.2; 32768x3584 W8A16
-// 35.2 / 27.4 / 52.8 (eight rows of four fp32-multiplied chunks do not fit the registers of two waves
-// per SIMD); 32768x1024 W8A16 12.8 / 15.9 / 41.1.
+// behind one another.  Measured on both sides of each line, us per call in a captured graph of 20 calls
+// on rotating weights, R = 8 / 4 / 1:
+//   rows     K = 1024 W8A8   W8A16            K = 3584 W8A8   W8A16
+//     512    3.6 / 3.1 / 3.4  4.3 / 3.7 / 3.7   5.6 / 4.5 / 3.9   7.4 / 5.6 / 4.4
+//    2048    4.0 / 3.7 / 3.8  4.5 / 3.9 / 4.2   5.9 / 4.9 / 5.0   7.6 / 5.9 / 5.5
+//    2056    4.0 / 3.6 / 3.9  4.4 / 3.9 / 5.2   6.0 / 4.8 / 5.2   7.6 / 5.9 / 7.1
+//    4096    4.1 / 3.9 / 4.7  4.6 / 4.2 / 6.7   6.7 / 6.0 / 7.7   8.2 / 6.8 / 9.2
+//    4104    4.1 / 3.9 / 4.7  4.6 / 4.3 / 7.4   6.6 / 8.1 / 7.7   8.1 / 7.5 / 10.0
+//    8192    4.5 / 4.5 / 7.1  5.0 / 5.0 / 11.7  7.8 / 9.8 / 11.7  9.7 / 8.8 / 15.7
+//    8200    4.6 / 4.5 / 7.0  5.1 / 6.0 / 11.9  11.1 / 11.9 / 11.7  14.7 / 10.5 / 15.8
+//   32768    9.1 / 9.8 / 19.6  11.2 / 14.0 / 39.4  25.8 / 32.4 / 36.6  33.1 / 25.5 / 51.0
+// and at the line in K, 32768 rows: K = 2048 W8A8 14.1 / 15.0, W8A16 15.4 / 18.7; K = 2064 W8A8 19.2 /
+// 18.1, W8A16 25.1 / 20.3 (past two chunks, eight rows of fp32-multiplied chunks do not fit the registers
+// of two waves per SIMD).
 int gemv_rows(int rows, int K, int mode) {
   if (rows <= 2048) return 1;
   if (K > 2048) return mode == M_W8A16 || rows <= 4096 ? 4 : 8;

@@ -1047,8 +1047,10 @@ hipError_t pf_norm(const PfNorm& a, int mode, hipStream_t s) {
 }
 
 namespace {
-// Token tiles per workgroup: as few as keep the grid within one round of two workgroups per CU
-// (a second, nearly empty round would cost as much as the first), at least `least`.
+// Token tiles per workgroup: as few as keep the grid within 512 workgroups, at least `least`.  512 is one
+// round of two workgroups per CU (a second, nearly empty round would cost as much as the first), which
+// is what fits for every product but the fp32 one with K = 3584: its 144 KiB of LDS leave one per CU, so
+// that at 768 tokens its 384 workgroups run in two rounds.
 int tiles_per_wg(int row_tiles, int ntile, int least) {
   const int ny = 512 / row_tiles > 0 ? 512 / row_tiles : 1;
   int t = (ntile + ny - 1) / ny;
