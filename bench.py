@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Batch-1 decode throughput of the 24-layer int8 hybrid model on one MI355X.
 
-Workload (BASELINE.json configs[4], "C5"): the full Qwen3.5-0.8B-shaped model
+Workload ("C5"): the full Qwen3.5-0.8B-shaped model
 with seeded synthetic int8 weights in the packed pack_weights.py layout; a
 64-token seeded prompt is fed (untimed; all but its last token as one group), then
 `--steps` greedy decode steps are timed (default 512, so the KV cache grows to
@@ -302,7 +302,7 @@ def config_profile():
 
 
 def op_configs(q, torch, np, blob, idx, act_mode, with_c4=True):
-    """BASELINE.json configs C1-C4, each unit's bytes the algorithmic count of the config
+    """The op configs C1-C4, each unit's bytes the algorithmic count of the config
     (weights + scales + activations + state / cache traffic).  C1-C3 run the op-level C ABI with
     no allocation inside a timed call (C2 and C3 take their scratch from a workspace / the
     library's static array) and rotate through > 256 MB of weights, states and caches, so no
@@ -497,7 +497,7 @@ def cpu_baseline(blob, idx, prompt, ntok, act_mode):
 
 
 def cpu_config_legs(blob, idx):
-    """BASELINE.json configs C1-C4 on one core, per unit: the reference's hls/src kernels
+    """The op configs C1-C4 on one core, per unit: the reference's hls/src kernels
     (oracle/_ref, compiled from the headers where they lie) built -O3 (`value`) and with the
     reference's csim flags, -O2 (`value_o2`), both -ffp-contract=off, W8A16 (the reference's own
     arithmetic).  C3 at T = 32768 exceeds the reference's sc[8192] bound (attention.hpp:66): that

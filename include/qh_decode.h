@@ -131,7 +131,7 @@ int qh_delta_rule_head(const float* q, const float* k, const float* v, float g, 
 int qh_delta_rule_layer(const float* q, const float* k, const float* v, const float* g,
                         const float* beta, float* S, float* out, void* stream);
 /* the DeltaNet recurrent step between the projections       deltanet.hpp:154-179 (inside deltanet_layer)
- * short conv + SiLU over the projected qkv [6144] (conv_state [6144][4] and
+ * (config C2): short conv + SiLU over the projected qkv [6144] (conv_state [6144][4] and
  * rec [16][128][128] updated in place), beta = sigmoid(b), g = -exp(A_log) softplus(a + dt_bias),
  * l2norm of q and k, q / sqrt(128), the delta rule, per-head gated RMSNorm with silu(z [2048]):
  * out [2048] (the input of out_proj).  The reference has no separate entry for this step; it is

@@ -53,7 +53,7 @@ void ref_conv1d_step(float* out, const float* in, float* state, const float* w) 
   conv1d_step(out, in, reinterpret_cast<float(*)[CONV_K]>(state), w);
 }
 void ref_rope_cos_sin(int pos, float* c, float* s) { rope_cos_sin(pos, c, s); }
-// The recurrent step between deltanet_layer's projections, from the
+// The recurrent step between deltanet_layer's projections (config C2), from the
 // reference's own functions in deltanet_layer's order (deltanet.hpp:154-179): conv1d_step,
 // the gates, l2norm and q scaling, delta_rule_layer, per-head rmsnorm_gated.
 void ref_deltanet_step(float* og, const float* qkv, const float* z, const float* b, const float* a,

@@ -1,5 +1,5 @@
 """How far from the reference's numpy golden (golden/model.py) each golden stage lands, against the
-north_star's literal tolerance, rtol 1e-4 / atol 1e-5 elementwise, for two implementations:
+literal tolerance of rtol 1e-4 / atol 1e-5 elementwise, for two implementations:
 
   device     the device-order twin (oracle.c ORDER_DEV), bit for bit the HIP path (the GPU tests
              compare them per op, per layer and per decode step);
